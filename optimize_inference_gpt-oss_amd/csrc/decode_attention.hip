@@ -34,8 +34,9 @@
 //            index b + w (unique: ranges are contiguous).
 //   combine  one workgroup per range: the range's split launch (or the prep
 //            launch) recorded the sequence the range starts inside of; the
-//            first range inside a sequence merges its partials with the
-//            sink. Empty sequences get zeros from the split (or prep) launch.
+//            first range inside a sequence (or, for a sequence in many
+//            pieces, every range inside it, the kv heads dealt over them)
+//            merges its partials with the sink. Empty sequences get zeros from the split (or prep) launch.
 //
 // Matrix cores: v_mfma_f32_16x16x32_bf16, 16x16 output, K = 32.
 //   scores  S^T[token][col] = K[token][dims] * Q^T[dims][col]      (2 MFMAs per 16 tokens)
@@ -140,7 +141,7 @@ struct DecodeArgs {
   float *ws_o;        // [range][kPartsPerRange][Hkv][8][64]: partial outputs
   float *ws_ml;       // [range][kPartsPerRange][Hkv][8][2]: their (m, l)
   int4 *crec;         // [range]: the combine's record ({b, w0, w1, cu[b]} of the sequence the
-                      // range is the first to start inside of; b = -1: none)
+                      // range starts inside of and merges a part of; b = -1: none)
   void *out;
   int64_t out_stride;
   int out_bf16;
@@ -214,15 +215,24 @@ __device__ __forceinline__ u32x2 int8x4_to_bf16x4(uint32_t w) {
   return u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
 }
 
-// The combine's record for range w, which starts at stream position rs and
-// inside sequence b ([c0, c1) of the stream; b = -1: at a sequence's start or
-// past the stream): the sequence's pieces are in ranges w0 = w - 1 .. w1,
-// and range w merges them if it is the first range to start inside it.
+// Sequences in at most this many pieces are merged by one workgroup, a wave
+// per kv head, every piece's loads at once; longer ones are spread over the
+// workgroups of the ranges that start inside of them.
+constexpr int kCombineAtOnce = 4;
+
+// The combine's record for range w, which starts inside sequence b ([c0, c1)
+// of the stream; b = -1: at a sequence's start or past the stream): the
+// sequence's pieces are in ranges w0 .. w1. A sequence of at most
+// kCombineAtOnce pieces is merged by the first range that starts inside it,
+// a longer one by all of them (every record is left).
 __device__ __forceinline__ int4 combine_record(int w, int b, int c0, int c1, int T, int S,
                                                int n) {
-  if (b < 0 || w == 0 || range_start(w - 1, T, S, n) > c0)
+  if (b < 0 || w == 0)
     return int4{-1, 0, 0, 0};
-  return int4{b, w - 1, range_of(c1 - 1, T, S, n), c0};
+  const int w0 = range_of(c0, T, S, n), w1 = range_of(c1 - 1, T, S, n);
+  if (w1 - w0 < kCombineAtOnce && w != w0 + 1)
+    return int4{-1, 0, 0, 0};
+  return int4{b, w0, w1, c0};
 }
 
 // ---- prep -----------------------------------------------------------------------
@@ -1437,97 +1447,174 @@ void decode_fused_kernel(DecodeArgs a, AppendArgs ap, int mode) {
 // ---- combine --------------------------------------------------------------------
 
 // Sequence b's output from its pieces in ranges w0 .. w1 (the stream
-// positions [c0, c1) meet them), one wave per kv head g; lane (h = lane / 8)
-// merges dims 8*(lane % 8) .. +7 of query head h:
+// positions [c0, c1) meet them):
 // M = max(sink, m_w), L = 2^(sink-M) + sum l_w 2^(m_w-M), out = sum o_w 2^(m_w-M) / L
 // (the merge of fast_attention.hpp:403-424, across workgroups). The piece in
 // range w is that range's last segment (slot 1) for the first range unless
 // the sequence starts exactly there, else its first segment (slot 0); ranges
 // without tokens (possible when there are fewer steps than ranges) hold none.
-// Up to kCombineAtOnce ranges, every load goes out at once (one round trip).
-constexpr int kCombineAtOnce = 4;
+// In both forms lane (h = lane / 8) of a wave holds dims 8*(lane % 8) .. +7 of
+// query head h of one kv head.
+__device__ __forceinline__ int64_t partial_index(const DecodeArgs &a, int4 rec, int r, int rs,
+                                                 int g) {
+  const int slot = (r == rec.y && rec.w != rs) ? 1 : 0;
+  return ((int64_t)r * kPartsPerRange + slot) * a.n_kv_heads + g;
+}
+
+// At most kCombineAtOnce pieces: one wave per kv head, every load at once.
 __device__ __forceinline__ void combine_sequence(const DecodeArgs &a, int4 rec) {
   constexpr int D = kHeadDim;
   const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, h = lane >> 3, d0 = 8 * (lane & 7);
-  if (h >= a.G)
+  if (h >= a.G || g >= a.n_kv_heads)
     return;
-  const int b = rec.x, w0 = rec.y, w1 = rec.z, c0 = rec.w;
+  const int b = rec.x, w0 = rec.y, w1 = rec.z;
   const int32_t *rsa = a.plan + kPlanHeader + a.B + 1 + a.n_wg; // range starts (+ the end)
-  auto part_of = [&](int r, int rs) -> int64_t {
-    const int slot = (r == w0 && c0 != rs) ? 1 : 0;
-    return ((int64_t)r * kPartsPerRange + slot) * a.n_kv_heads + g;
-  };
   const int64_t ob = (int64_t)b * a.out_stride + (int64_t)(g * a.G + h) * D + d0;
   const float sk = a.sinks[g * a.G + h] * kLog2e;
-  float M = sk, Ls, inv;
+  float M = sk;
   f32x4 o0 = {0, 0, 0, 0}, o1 = {0, 0, 0, 0};
-  if (w1 - w0 < kCombineAtOnce) {
-    float m[kCombineAtOnce], l[kCombineAtOnce];
-    f32x4 pa[kCombineAtOnce], pb[kCombineAtOnce];
-    bool ok[kCombineAtOnce];
+  float m[kCombineAtOnce], l[kCombineAtOnce];
+  f32x4 pa[kCombineAtOnce], pb[kCombineAtOnce];
+  bool ok[kCombineAtOnce];
 #pragma unroll
-    for (int i = 0; i < kCombineAtOnce; i++) {
-      const int r = w0 + i;
-      ok[i] = false;
-      if (r <= w1) {
-        const int rs = rsa[r];
-        ok[i] = rs != rsa[r + 1];
-        const int64_t part = part_of(r, rs);
-        m[i] = a.ws_ml[part * kMlStride + 2 * h];
-        l[i] = a.ws_ml[part * kMlStride + 2 * h + 1];
-        const f32x4 *po = (const f32x4 *)(a.ws_o + part * kPartFloats + h * D + d0);
-        pa[i] = po[0];
-        pb[i] = po[1];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kCombineAtOnce; i++)
-      if (ok[i])
-        M = fmaxf(M, m[i]);
-    Ls = __builtin_amdgcn_exp2f(sk - M);
-#pragma unroll
-    for (int i = 0; i < kCombineAtOnce; i++)
-      if (ok[i]) {
-        const float c = __builtin_amdgcn_exp2f(m[i] - M);
-        Ls = fmaf(l[i], c, Ls);
-        o0 += pa[i] * c;
-        o1 += pb[i] * c;
-      }
-  } else {
-    for (int r = w0; r <= w1; r++)
-      if (rsa[r] != rsa[r + 1])
-        M = fmaxf(M, a.ws_ml[part_of(r, rsa[r]) * kMlStride + 2 * h]);
-    Ls = __builtin_amdgcn_exp2f(sk - M);
-    for (int r = w0; r <= w1; r++) {
-      if (rsa[r] == rsa[r + 1])
-        continue;
-      const int64_t part = part_of(r, rsa[r]);
-      const float c = __builtin_amdgcn_exp2f(a.ws_ml[part * kMlStride + 2 * h] - M);
-      Ls = fmaf(a.ws_ml[part * kMlStride + 2 * h + 1], c, Ls);
+  for (int i = 0; i < kCombineAtOnce; i++) {
+    const int r = w0 + i;
+    ok[i] = false;
+    if (r <= w1) {
+      const int rs = rsa[r];
+      ok[i] = rs != rsa[r + 1];
+      const int64_t part = partial_index(a, rec, r, rs, g);
+      m[i] = a.ws_ml[part * kMlStride + 2 * h];
+      l[i] = a.ws_ml[part * kMlStride + 2 * h + 1];
       const f32x4 *po = (const f32x4 *)(a.ws_o + part * kPartFloats + h * D + d0);
-      o0 += po[0] * c;
-      o1 += po[1] * c;
+      pa[i] = po[0];
+      pb[i] = po[1];
     }
   }
-  inv = 1.0f / Ls;
+#pragma unroll
+  for (int i = 0; i < kCombineAtOnce; i++)
+    if (ok[i])
+      M = fmaxf(M, m[i]);
+  float Ls = __builtin_amdgcn_exp2f(sk - M);
+#pragma unroll
+  for (int i = 0; i < kCombineAtOnce; i++)
+    if (ok[i]) {
+      const float c = __builtin_amdgcn_exp2f(m[i] - M);
+      Ls = fmaf(l[i], c, Ls);
+      o0 += pa[i] * c;
+      o1 += pb[i] * c;
+    }
+  const float inv = 1.0f / Ls;
   for (int i = 0; i < 4; i++) {
     store_out(a.out, ob + i, o0[i] * inv, a.out_bf16);
     store_out(a.out, ob + 4 + i, o1[i] * inv, a.out_bf16);
   }
 }
 
-// One workgroup per range, a wave per kv head: the split launch (or the
-// prepare launch of the staged ones) left, per range, the record of the
-// sequence the range is the first to start inside of (its pieces' ranges and
-// stream start), so the merge is two round trips: the record, then every
-// piece at once. n_wg workgroups instead of one per sequence, most of them
-// returning at once.
-__global__ __launch_bounds__(512) void decode_combine_kernel(DecodeArgs a) {
+// More pieces (few long sequences, cut into many short ranges): one kv head
+// by a whole workgroup. Wave v merges pieces w0 + v, w0 + v + 8, ..., four
+// loaded at a time (their loads do not depend on each other; the partial of a
+// range without tokens is read like the others and left out), then the waves'
+// results meet in LDS in wave order.
+constexpr int kCombineWaves = 8;
+__device__ __forceinline__ void combine_head_wide(const DecodeArgs &a, int4 rec, int g) {
+  constexpr int D = kHeadDim;
+  __shared__ f32x4 s_o[kCombineWaves][64][2];
+  __shared__ float2 s_ml[kCombineWaves][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, d0 = 8 * (lane & 7);
+  const bool head_ok = (lane >> 3) < a.G;
+  const int h = head_ok ? lane >> 3 : 0;
+  const int b = rec.x, w0 = rec.y, w1 = rec.z;
+  const int32_t *rsa = a.plan + kPlanHeader + a.B + 1 + a.n_wg;
+  const float sk = a.sinks[g * a.G + h] * kLog2e;
+  const int rs0 = rsa[w0];
+  float M = sk, Ls = 0.0f; // (the sink's own weight is added at the end)
+  f32x4 o0 = {0, 0, 0, 0}, o1 = {0, 0, 0, 0};
+  for (int r0 = w0 + wave; r0 <= w1; r0 += 4 * kCombineWaves) {
+    float m[4], l[4];
+    f32x4 pa[4], pb[4];
+    bool ok[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int r = min(r0 + i * kCombineWaves, w1);
+      const int64_t part = partial_index(a, rec, r, rs0, g);
+      ok[i] = r0 + i * kCombineWaves <= w1 && rsa[r] != rsa[r + 1];
+      const float2 ml = *(const float2 *)&a.ws_ml[part * kMlStride + 2 * h];
+      m[i] = ml.x;
+      l[i] = ml.y;
+      const f32x4 *po = (const f32x4 *)(a.ws_o + part * kPartFloats + h * D + d0);
+      pa[i] = po[0];
+      pb[i] = po[1];
+    }
+    float Mn = M;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (ok[i])
+        Mn = fmaxf(Mn, m[i]);
+    const float c0 = __builtin_amdgcn_exp2f(M - Mn);
+    M = Mn;
+    Ls *= c0;
+    o0 *= c0;
+    o1 *= c0;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (ok[i]) {
+        const float c = __builtin_amdgcn_exp2f(m[i] - M);
+        Ls = fmaf(l[i], c, Ls);
+        o0 += pa[i] * c;
+        o1 += pb[i] * c;
+      }
+  }
+  __syncthreads(); // (the arrays may still be read for another head)
+  s_o[wave][lane][0] = o0;
+  s_o[wave][lane][1] = o1;
+  s_ml[wave][lane] = float2{M, Ls};
+  __syncthreads();
+  if (wave != 0 || !head_ok)
+    return;
+  float Mt = sk;
+#pragma unroll
+  for (int v = 0; v < kCombineWaves; v++)
+    Mt = fmaxf(Mt, s_ml[v][lane].x);
+  float Lt = __builtin_amdgcn_exp2f(sk - Mt);
+  o0 = o1 = f32x4{0, 0, 0, 0};
+#pragma unroll
+  for (int v = 0; v < kCombineWaves; v++) {
+    const float2 ml = s_ml[v][lane];
+    const float c = __builtin_amdgcn_exp2f(ml.x - Mt);
+    Lt = fmaf(ml.y, c, Lt);
+    o0 += s_o[v][lane][0] * c;
+    o1 += s_o[v][lane][1] * c;
+  }
+  const float inv = 1.0f / Lt;
+  const int64_t ob = (int64_t)b * a.out_stride + (int64_t)(g * a.G + h) * D + d0;
+  for (int i = 0; i < 4; i++) {
+    store_out(a.out, ob + i, o0[i] * inv, a.out_bf16);
+    store_out(a.out, ob + 4 + i, o1[i] * inv, a.out_bf16);
+  }
+}
+
+// One workgroup per range: the split launch (or the prepare launch of the
+// staged ones) left, per range, the record of the sequence that it starts
+// inside of. Bound by latency: the record, the range starts, then the pieces.
+// A sequence of at most kCombineAtOnce pieces is merged by one workgroup (the
+// others of its ranges return at once); the kv heads of a longer one are
+// dealt over the workgroups of all the ranges that start inside of it. (One
+// workgroup going through 64 pieces in order, a round trip each, took 41.9 us
+// for 4 sequences of 129 .. 2049 tokens in 256 ranges; spread: 8.5 us.)
+__global__ __launch_bounds__(64 * kCombineWaves) void decode_combine_kernel(DecodeArgs a) {
   const int4 rec = a.crec[blockIdx.x];
   if (rec.x < 0)
     return;
-  combine_sequence(a, rec);
+  const int n_inside = rec.z - rec.y; // ranges w0 + 1 .. w1 start inside the sequence
+  if (n_inside < kCombineAtOnce) {
+    combine_sequence(a, rec);
+    return;
+  }
+  for (int g = (int)blockIdx.x - rec.y - 1; g < a.n_kv_heads; g += n_inside)
+    combine_head_wide(a, rec, g);
 }
 
 // ---- host side --------------------------------------------------------------------
@@ -1839,7 +1926,7 @@ static int launch_fused(const DecodeArgs &a, const AppendArgs *ap, hipStream_t s
 }
 
 static int launch_combine(const DecodeArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL(decode_combine_kernel, dim3(a.n_wg), dim3(64 * a.n_kv_heads), 0, s, a);
+  hipLaunchKernelGGL(decode_combine_kernel, dim3(a.n_wg), dim3(64 * kCombineWaves), 0, s, a);
   return launch_status("decode_combine_kernel");
 }
 

@@ -202,6 +202,24 @@ def test_split_sizes_agree(gkv, cuda, torch_mod, split_tokens):
     check_case(case, run_gpu(case, gkv, torch_mod, cuda, split_tokens=split_tokens))
 
 
+@pytest.mark.parametrize("heads", [(64, 8), (6, 2), (5, 1)])
+def test_combine_of_many_pieces(gkv, cuda, torch_mod, heads):
+    # ranges of 32 tokens: sequences of 1 .. 4 pieces (merged by one workgroup),
+    # 5 and 6 (more kv heads than ranges inside), 8 x 4 +- 1 (one batch of
+    # loads per wave, and one more), and 76
+    L = np.array([0, 31, 63, 64, 127, 128, 159, 991, 1023, 1055, 2431, 40], np.int32)
+    case = DecodeCase(len(L), heads[0], heads[1], L, window=0, seed=29, scale=0.7)
+    check_case(case, run_gpu(case, gkv, torch_mod, cuda, split_tokens=32))
+
+
+@pytest.mark.parametrize("lens", [[40], [4095], [1500, 0, 2, 700]])
+def test_few_sequences_in_more_ranges_than_steps(gkv, cuda, torch_mod, lens):
+    # a balanced split of fewer 32-token steps than ranges: ranges without
+    # tokens lie between the pieces
+    case = DecodeCase(len(lens), 64, 8, np.array(lens, np.int32), window=0, seed=31)
+    check_case(case, run_gpu(case, gkv, torch_mod, cuda))
+
+
 def test_rotated_q_path_and_bf16_output(gkv, cuda, torch_mod):
     L = np.array([3, 200, 900, 64], np.int32)
     case = DecodeCase(len(L), 64, 8, L, window=0, scale=0.5, seed=66)
