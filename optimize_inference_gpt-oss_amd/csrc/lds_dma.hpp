@@ -70,6 +70,27 @@ __device__ __forceinline__ void dma16_s(const void *base, uint32_t byte_off, voi
                : "memory");
 }
 
+// dma16_s in a loop whose LDS and global addresses are kept as numbers: the
+// LDS byte address of the wave's 1 KB (the low half of a generic pointer into
+// LDS is its LDS address) and the base both wave-uniform. M0 is declared
+// overwritten instead of saved, so the load is three instructions.
+__device__ __forceinline__ uint32_t lds_addr(const void *p) {
+  return (uint32_t)(uintptr_t)(lds_ptr)p;
+}
+__device__ __forceinline__ void dma16_at(const void *base, uint32_t byte_off, uint32_t lds) {
+  const uint64_t b = (uint64_t)(uintptr_t)base;
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
+  const uint64_t sb = ((uint64_t)hi << 32) | lo;
+  const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane(lds);
+  asm volatile("s_mov_b32 m0, %2\n\t"
+               "s_nop 0\n\t"
+               "global_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(byte_off), "s"(sb), "s"(m)
+               : "memory", "m0");
+}
+
 // 4 bytes per lane straight into LDS: lane l's dword lands at l_base + 4 l.
 __device__ __forceinline__ void dma4(const void *src, void *l_base) {
   const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)l_base);

@@ -11,15 +11,22 @@
 // gemm_bf16 writes) are stored too when asked: the attention reads Q from
 // them.
 //
-// Work: one workgroup per kQkvBM x kQkvBN output tile (as built 64 x 64, one
-// head, 4 waves; three workgroups per CU), the K dimension in chunks of 64
-// through a 3-stage LDS pipeline fed by direct-to-LDS loads (16-byte slots
-// XOR-swizzled per row, as in the prefill kernel). Each wave owns 16 rows
-// (kRT row tiles of 16) and one head of the tile: kRT x 4 tiles of
-// v_mfma_f32_16x16x32_bf16, so a lane holds dims d and d + 32 of its rows --
-// both halves of a RoPE pair -- in registers. With the number of column
-// blocks a multiple of 8, the row blocks of one column block run on one XCD
-// (their W tile is read from one L2).
+// Work: one workgroup per output tile (shapes and the rule that picks one:
+// qkv_shape below), the K dimension in stages of one or more 64-wide pieces,
+// fed by direct-to-LDS loads (16-byte slots XOR-swizzled per row, as in the
+// prefill kernel). A wave owns some row tiles of 16 and one head of the tile
+// (and, where the rows are few, every kWK-th 32-wide K slice):
+// v_mfma_f32_16x16x32_bf16 with W as the first operand, so a lane holds 4
+// consecutive dims of one row (16-byte stores of the fp32 rows), d and d + 32
+// alike -- both halves of a RoPE pair. The operands of a slice are read from
+// LDS into registers among the matrix ops of the slice before, and one
+// barrier per stage both publishes the next stage and frees this one.
+// What bounds it: with many rows the matrix cores (9507 rows: 243 us = 1154
+// TFLOP/s, of which 200 in the K loop, the fp32 rows' 195 MB most of the rest;
+// 128 x 128 tiles without the operand buffering, the workgroups of an XCD
+// spread over all row blocks: 402), at 512 rows the latency of the operand
+// stream (1.2 us from a load's issue to its data, whatever the tile), with few
+// rows the chain of K steps.
 //
 // Placement of each row (its sequence, position, slot and block) is loaded by
 // the first waves in three dependent hops of direct-to-LDS loads spread over the
@@ -29,21 +36,10 @@
 #include "kv_append.hpp"
 #include "lds_dma.hpp"
 
-namespace gkv {
+#include <algorithm>
+#include <type_traits>
 
-// Launch shapes: output rows per workgroup (64 or 128), output columns (64 or
-// 128: one or two heads), the K chunk of a pipeline stage (32 or 64), the
-// LDS stages and the waves per workgroup. Few rows (a decode step): 64 x 64
-// tiles, three workgroups per CU, enough of them to fill the GPU. Many rows
-// (prompts): 128 x 128 tiles with 8 waves and 2 stages (two workgroups per
-// CU), four times the reuse of each loaded byte.
-constexpr int kQkvBM = 64;
-constexpr int kQkvWaves = 4;
-constexpr int kQkvBN = 64;
-constexpr int kQkvBK = 64;
-constexpr int kQkvStages = 3;
-constexpr int kQkvBigRows = 2048; // from this many rows on, the large tiles
-constexpr int kQkvBigBM = 128, kQkvBigBN = 128, kQkvBigWaves = 8, kQkvBigStages = 2;
+namespace gkv {
 
 struct QkvArgs {
   const uint16_t *x; // bf16 [M][x_stride]
@@ -52,106 +48,61 @@ struct QkvArgs {
   const float *bias; // [N] or nullptr
   float *out;        // fp32 [M][out_stride] or nullptr
   int64_t out_stride;
-  int M, N, K, m_blocks, xcd_map;
+  int M, N, K, m_blocks, n_blocks;
   AppendArgs ap; // placement, tables and cache of the append (qkv/q_out/packs unused)
 };
 
-template <int kGM, int kGN, int kGK, int kGStages, int kNW>
-__global__ __launch_bounds__(64 * kNW) void qkv_append_kernel(QkvArgs a) {
-  constexpr int kWN = kGN / 64;                // waves along N (one head each)
-  constexpr int kWM = kNW / kWN;               // waves along M
-  constexpr int kRT = kGM / 16 / kWM;          // 16-row tiles per wave
-  constexpr int kSPR = kGK / 8;                // 16-byte slots per row of a stage
-  constexpr int kRPC = 64 / kSPR;              // rows per 1 KB direct-to-LDS load
-  constexpr int kXChunks = kGM / kRPC / kNW;   // x loads per wave per chunk
-  constexpr int kWChunks = kGN / kRPC / kNW;   // W loads per wave per chunk
-  static_assert(kRT >= 1 && kXChunks >= 1 && kWChunks >= 1, "launch shape");
-  constexpr int kGPer = kXChunks + kWChunks;   // direct-to-LDS loads per wave per chunk
-  // slot swizzle of row r: 8 rows (64-wide chunk) or 4 row groups of 4
-  // (32-wide chunk) see every slot, so the 16 lanes reading one slot column of
-  // 16 rows hit distinct banks
-  auto swz = [](int r) { return kGK == 64 ? (r & 7) : ((r >> 2) & 3); };
-  __shared__ __attribute__((aligned(16))) uint16_t x_st[kGStages][kGM * kGK];
-  __shared__ __attribute__((aligned(16))) uint16_t w_st[kGStages][kGN * kGK];
-  __shared__ int s_pos[kGM], s_off[kGM];
-  __shared__ int64_t s_base[kGM];
-  // placement loads land here (direct-to-LDS, one int per row)
-  __shared__ __attribute__((aligned(16))) int s_seq[kGM], s_rpos[kGM], s_len[kGM], s_id[kGM];
+// Four floats at any float's alignment: this entry point asks none of the
+// output rows, the bias and the angle tables.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
-  const int n = lane & 15, kg = lane >> 4;
-  int mb, nb;
-  {
-    const int id = blockIdx.x;
-    if (a.xcd_map) { // the m blocks of column block nb on XCD nb % 8
-      const int x = id % 8, r = id / 8;
-      mb = r % a.m_blocks;
-      nb = x + 8 * (r / a.m_blocks);
-    } else {
-      mb = id % a.m_blocks;
-      nb = id / a.m_blocks;
-    }
+constexpr int kQkvBK = 64; // K per pipeline stage: 128 bytes of a row, 8 slots of 16 bytes
+
+// The 16-byte slot of stage row r that holds K piece s (8 values): 8 rows see
+// every slot, so the 16 lanes reading one piece of 16 rows hit distinct banks.
+__device__ __forceinline__ int qkv_slot(int r, int s) { return s ^ (r & 7); }
+
+// Row placement in the paged cache: the rows' sequence, position, slot and
+// block, one row per lane of the first waves (row 64 * wave + lane of the
+// tile), as three dependent hops of direct-to-LDS loads issued among the main
+// loop's (a register load would be left in flight across code the compiler
+// schedules freely).
+template <int kGM>
+struct QkvPlace {
+  static constexpr int kRows = (kGM + 63) / 64 * 64; // 64 per placing wave
+  int *s_seq, *s_rpos, *s_len, *s_id; // kRows ints each, 16-byte aligned
+  int *s_pos, *s_off;
+  int64_t *s_base;
+  int m0, wave, prl, pr;
+  bool place, need_len;
+  int p_slot = 0, p_pos = 0;
+  bool p_store = false;
+
+  __device__ __forceinline__ int row_seq_of(const AppendArgs &ap) const {
+    return ap.row_seq ? s_seq[prl] : pr;
   }
-  const int m0 = mb * kGM, n0 = nb * kGN;
-  const int nk = a.K / kGK;
-  const AppendArgs &ap = a.ap;
-  const bool appends = ap.kc != nullptr;
-
-  // ---- pipeline of K chunks; a chunk past the last re-reads the last one,
-  // so every iteration issues the same loads and the waits are exact.
-  auto dma = [&](int kc, int st) {
-    const int k0 = min(kc, nk - 1) * kGK;
-#pragma unroll
-    for (int i = 0; i < kXChunks; i++) {
-      const int c = wave + kNW * i;
-      const int r = c * kRPC + lane / kSPR, slot = lane % kSPR;
-      const int row = min(m0 + r, a.M - 1);
-      dma16(a.x + (int64_t)row * a.x_stride + k0 + 8 * (slot ^ swz(r)), &x_st[st][c * 512]);
-    }
-#pragma unroll
-    for (int i = 0; i < kWChunks; i++) {
-      const int c = wave + kNW * i;
-      const int r = c * kRPC + lane / kSPR, slot = lane % kSPR;
-      const int col = min(n0 + r, a.N - 1);
-      dma16(a.w + (int64_t)col * a.K + k0 + 8 * (slot ^ swz(r)), &w_st[st][c * 512]);
-    }
-  };
-
-  // ---- row placement (waves 0 .. kGM/64 - 1; lane t of wave w: row
-  // m0 + 64 w + t): hop 1 loads the row's sequence and position, hop 2
-  // its sequence length, hop 3 its block id, each a direct-to-LDS load (a
-  // register load would be left in flight across code the compiler schedules
-  // freely); hops 2 and 3 are issued inside the main loop after waits that
-  // cover the hop before.
-  const int prl = 64 * wave + lane; // row within the tile
-  const int pr = min(m0 + prl, a.M - 1);
-  const bool place = wave < kGM / 64 && appends;
-  const bool need_len = ap.seq_lens && (!ap.row_pos || ap.ring > 0);
-  auto place_hop1 = [&]() {
+  __device__ __forceinline__ void hop1(const AppendArgs &ap) {
     if (!place)
       return;
     if (ap.row_seq)
       dma4(ap.row_seq + pr, s_seq + 64 * wave);
     if (ap.row_pos)
       dma4(ap.row_pos + pr, s_rpos + 64 * wave);
-  };
-  auto row_seq_of = [&]() { return ap.row_seq ? s_seq[prl] : pr; };
-  auto place_hop2 = [&]() {
+  }
+  __device__ __forceinline__ void hop2(const AppendArgs &ap) { // hop 1 has landed
     if (!place || !need_len)
       return;
-    dma4(ap.seq_lens + row_seq_of(), s_len + 64 * wave);
-  };
-  int p_slot = 0, p_pos = 0;
-  bool p_store = false;
-  auto place_hop3 = [&]() {
+    dma4(ap.seq_lens + row_seq_of(ap), s_len + 64 * wave);
+  }
+  __device__ __forceinline__ void hop3(const AppendArgs &ap, int M) { // hop 2 has landed
     if (!place)
       return;
-    const int seq = row_seq_of();
+    const int seq = row_seq_of(ap);
     const int len = need_len ? s_len[prl] : 0;
     const int pos = ap.row_pos ? s_rpos[prl] : len - 1;
     p_pos = pos;
     p_slot = ap.ring > 0 ? pos % ap.ring : pos;
-    p_store = m0 + prl < a.M && pos >= 0;
+    p_store = prl < kGM && m0 + prl < M && pos >= 0;
     if (p_store && ap.ring > 0 && ap.seq_lens && pos + ap.ring < len)
       p_store = false; // a later row of this call takes the ring slot
     const int blk = p_slot / kBlockTokens;
@@ -162,9 +113,9 @@ __global__ __launch_bounds__(64 * kNW) void qkv_append_kernel(QkvArgs a) {
     }
     // rows that are not stored load entry 0 (any valid address)
     dma4(ap.table + (p_store ? (int64_t)seq * ap.table_stride + blk : 0), s_id + 64 * wave);
-  };
-  auto place_finish = [&]() { // after the loop's final wait: every load has landed
-    if (wave >= kGM / 64)
+  }
+  __device__ __forceinline__ void finish(const AppendArgs &ap) { // every load has landed
+    if (wave >= kRows / 64)
       return;
     int64_t base = -1;
     if (place && p_store) {
@@ -179,10 +130,296 @@ __global__ __launch_bounds__(64 * kNW) void qkv_append_kernel(QkvArgs a) {
     s_pos[prl] = max(p_pos, 0);
     s_off[prl] = base >= 0 ? p_slot % kBlockTokens : -1;
     s_base[prl] = base;
+  }
+};
+
+// Staged V rows: row r of a wave (its 64 values of one head) in LDS as bf16, or
+// as codes of one byte. The 16-byte slots of a bf16 row (8 slots) and the
+// 8-byte ones of a row of codes are XOR-swizzled by the row, so that the 16
+// lanes writing one piece of 16 rows spread over the banks.
+__device__ __forceinline__ int v_stage_bf16(int r, int d) { // element offset
+  return r * 64 + 8 * ((d >> 3) ^ (r & 7)) + (d & 7);
+}
+__device__ __forceinline__ int v_stage_code(int r, int d) { // byte offset
+  return r * 64 + 8 * ((d >> 3) ^ (r & 7)) + (d & 7);
+}
+
+// One row tile of 16 rows x one head from its finished sums: lane (kg, n)
+// holds row m (lr within the workgroup's tile), dims 16 j + 4 kg + r in
+// acc[j][r], both halves (d, d + 32) of its RoPE pairs. Adds the bias, stores
+// the fp32 row; a K head goes into the cache exactly as gkv_kv_append rounds
+// and places it, a V head's cache values into vst (the wave's staged rows, row
+// vr) for qkv_store_values.
+template <int kGM>
+__device__ __forceinline__ void qkv_store_row(const QkvArgs &a, const QkvPlace<kGM> &pl,
+                                              f32x4 (&acc)[4], const f32x4 (&bias)[4], int hd,
+                                              int lr, int kg, char *vst, int vr) {
+  constexpr int D = kHeadDim, HALF = kHeadDim / 2;
+  const AppendArgs &ap = a.ap;
+  const int m = pl.m0 + lr, c0 = D * hd + 4 * kg;
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    acc[j] += bias[j];
+  if (a.out && m < a.M) {
+    float *o = a.out + (int64_t)m * a.out_stride + c0;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      *(f32x4u *)(o + 16 * j) = acc[j];
+  }
+  if (!ap.kc || hd < ap.n_q_heads)
+    return;
+  const bool is_k = hd < ap.n_q_heads + ap.n_kv_heads;
+  const int g = is_k ? hd - ap.n_q_heads : hd - ap.n_q_heads - ap.n_kv_heads;
+  const int off = pl.s_off[lr];
+  const int64_t base = pl.s_base[lr] + (int64_t)g * (kBlockTokens * D);
+  const bool st_ok = off >= 0; // (rows past the last have none)
+  f32x4 y[4];
+  if (is_k) {
+    const int pos = pl.s_pos[lr];
+#pragma unroll
+    for (int j = 0; j < 2; j++) { // dims 16 j + 4 kg .. +3 and those + 32
+      const f32x4 c = *(const f32x4u *)(ap.cos_tab + (int64_t)pos * HALF + 16 * j + 4 * kg);
+      const f32x4 s = *(const f32x4u *)(ap.sin_tab + (int64_t)pos * HALF + 16 * j + 4 * kg);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        y[j][r] = rope_first(acc[j][r], acc[j + 2][r], c[r], s[r]);
+        y[j + 2][r] = rope_second(acc[j][r], acc[j + 2][r], c[r], s[r]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      y[j] = acc[j];
+  }
+  const bool quant = ap.kv_fp8 || (ap.v_int8 && !is_k);
+  uint32_t code[4]; // of dims 16 j + 4 kg .. +3
+  if (quant) {
+    float amax = 0.0f; // of the head's 64 dims: 16 in this lane, 4 lanes
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        amax = fmaxf(amax, fabsf(y[j][r]));
+    amax = fmaxf(amax, __shfl_xor(amax, 16));
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    if (ap.kv_fp8) {
+      // e4m3: one scale per token and head (K's, then V's)
+      const float inv = amax > 0.0f ? 448.0f / amax : 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        code[j] = fp8x4(y[j][0], y[j][1], y[j][2], y[j][3], inv);
+      if (st_ok && kg == 0)
+        ap.vs[base / 32 + (is_k ? 0 : kBlockTokens) + off] = amax / 448.0f;
+    } else {
+      // the reference's rule, getp-csrc/kernels/fast_misc.hpp:74-84
+      const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        code[j] = 0;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float cq = fminf(fmaxf(rintf(y[j][r] * inv), -127.0f), 127.0f);
+          code[j] |= (uint32_t)(uint8_t)(int8_t)cq << (8 * r);
+        }
+      }
+      if (st_ok && kg == 0)
+        ap.vs[base / D + off] = amax / 127.0f;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int d = 16 * j + 4 * kg;
+    const u32x2 w{f32_to_bf16_rne(y[j][0]) | ((uint32_t)f32_to_bf16_rne(y[j][1]) << 16),
+                  f32_to_bf16_rne(y[j][2]) | ((uint32_t)f32_to_bf16_rne(y[j][3]) << 16)};
+    if (!is_k && quant)
+      *(uint32_t *)(vst + v_stage_code(vr, d)) = code[j];
+    else if (!is_k)
+      *(u32x2 *)(vst + 2 * v_stage_bf16(vr, d)) = w;
+    else if (st_ok && quant)
+      *(uint32_t *)((uint8_t *)ap.kc + base + k_fp8_offset(off, d)) = code[j];
+    else if (st_ok)
+      *(u32x2 *)(ap.kc + base + k_offset(off, d)) = w;
+  }
+}
+
+// The staged V rows of one head (rows lr0 .. lr0 + n_rows - 1 of the tile, at
+// most 64, staged as rows 0 ..) into the cache, by one wave. Four rows holding
+// slots 4m .. 4m+3 of one block (consecutive tokens of a prompt) go together
+// as 16-byte pieces (bf16: dims d and d + 16 of the 4 tokens; codes: dims d,
+// d + 16, d + 32, d + 48); a row alone goes as one store of its 64 dims, whose
+// lanes then meet in few cache lines. (Stored straight from the matrix layout,
+// 16 rows x 4 dims an instruction, the V heads' workgroups took 7.5 us longer
+// than the others at 512 decode rows.)
+template <int kGM>
+__device__ __forceinline__ void qkv_store_values(const AppendArgs &ap, const QkvPlace<kGM> &pl,
+                                                 const char *vst, int lr0, int n_rows, int g,
+                                                 int lane) {
+  const bool code = ap.v_int8 || ap.kv_fp8;
+  const int64_t hb = (int64_t)g * (kBlockTokens * kHeadDim);
+  const int off = lane < n_rows ? pl.s_off[lr0 + lane] : -1;
+  bool lead = lane + 3 < n_rows && off >= 0 && (off & 3) == 0;
+#pragma unroll
+  for (int k = 1; k < 4; k++) {
+    const int r = min(lane + k, n_rows - 1) + lr0;
+    lead = lead && pl.s_off[r] == off + k && pl.s_base[r] == pl.s_base[lr0 + lane];
+  }
+  uint64_t quads = __ballot(lead);
+  uint64_t alone = __ballot(off >= 0) & ~(quads | quads << 1 | quads << 2 | quads << 3);
+  const int per = code ? 16 : 32; // lanes per quad
+  while (quads) {
+    int r0 = -1; // this lane's quad
+    for (int k = 0; k < 64 / per && quads; k++) {
+      const int r = __builtin_ctzll(quads);
+      quads &= quads - 1;
+      r0 = lane / per == k ? r : r0;
+    }
+    if (r0 < 0)
+      continue;
+    const int t0 = pl.s_off[lr0 + r0];
+    const int64_t base = pl.s_base[lr0 + r0] + hb;
+    if (code) {
+      const int d = lane & 15;
+      uint32_t w[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        w[q] = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          w[q] |= (uint32_t)(uint8_t)vst[v_stage_code(r0 + k, d + 16 * q)] << (8 * k);
+      }
+      *(u32x4 *)((uint8_t *)ap.vc + base + v_int8_offset(d, t0)) = u32x4{w[0], w[1], w[2], w[3]};
+    } else {
+      const int d = 32 * ((lane >> 4) & 1) + (lane & 15);
+      uint16_t h[8];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        h[k] = ((const uint16_t *)vst)[v_stage_bf16(r0 + k, d)];
+        h[4 + k] = ((const uint16_t *)vst)[v_stage_bf16(r0 + k, d + 16)];
+      }
+      *(u32x4 *)(ap.vc + base + v_offset(t0, d)) = pack8(h);
+    }
+  }
+  while (alone) {
+    const int r = __builtin_ctzll(alone);
+    alone &= alone - 1;
+    const int t = pl.s_off[lr0 + r];
+    const int64_t base = pl.s_base[lr0 + r] + hb;
+    if (code)
+      ((uint8_t *)ap.vc)[base + v_int8_offset(lane, t)] = (uint8_t)vst[v_stage_code(r, lane)];
+    else
+      ap.vc[base + v_offset(t, lane)] = ((const uint16_t *)vst)[v_stage_bf16(r, lane)];
+  }
+}
+
+// kGM x kGN output tile, kWM x (kGN / 64) x kWK waves, kSub 64-wide K pieces per
+// stage: wave (wm, wn, wk) sums rows [wm] of head [wn] over the 32-wide slices
+// wk, wk + kWK, .. of every stage; with kWK > 1 the sums of a tile meet in LDS
+// after the loop.
+template <int kGM, int kGN, int kWM, int kWK, int kSub, int kGStages, bool kWide = false>
+__global__ __launch_bounds__(64 * kWM * (kGN / 64) * kWK) void qkv_append_kernel(QkvArgs a) {
+  constexpr int kWN = kGN / 64, kNW = kWM * kWN * kWK;
+  constexpr int kRT = kGM / 16 / kWM;            // 16-row tiles per wave
+  constexpr int kSl = 2 * kSub / kWK;            // slices per wave and stage
+  constexpr int kXC = kGM / 8, kWC = kGN / 8;    // 1 KB direct-to-LDS loads per 64 of K: x, W
+  constexpr int kUnits = kSub * (kXC + kWC);
+  constexpr int kGPer = (kUnits + kNW - 1) / kNW; // per wave and stage
+  static_assert(kRT >= 1 && kGM % (16 * kWM) == 0 && (2 * kSub) % kWK == 0 &&
+                    kNW >= QkvPlace<kGM>::kRows / 64,
+                "launch shape");
+  static_assert((kWK - 1) * kGM * kGN * 4 <= kGStages * kSub * (kGM + kGN) * kQkvBK * 2 &&
+                    kGM * kGN * 2 * (kWK > 1 ? 2 : 1) <= kGStages * kSub * (kGM + kGN) * kQkvBK * 2,
+                "the slices' sums and the staged V rows fit the stages");
+  using Place = QkvPlace<kGM>;
+  constexpr int kSubElems = (kGM + kGN) * kQkvBK, kStageElems = kSub * kSubElems;
+  __shared__ __attribute__((aligned(16))) uint16_t stage[kGStages * kStageElems];
+  __shared__ __attribute__((aligned(16))) int s_place[6 * Place::kRows];
+  __shared__ int64_t s_base[Place::kRows];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+  const int n = lane & 15, kg = lane >> 4;
+  int mb, nb;
+  {
+    // workgroup id -> tile: the ids of one XCD (id % 8) take consecutive tiles,
+    // in groups of 8 row blocks x all column blocks, rows fastest, so that the
+    // tiles an XCD holds at once share their rows and columns in its L2. The
+    // columns go round the XCDs (column c of an XCD's n / 8 is block 8 c + its
+    // index), from the last one down: the K and V heads, whose epilogue is
+    // longer, are spread over all XCDs and start first.
+    const int x = blockIdx.x % 8, q = gridDim.x / 8, rem = gridDim.x % 8;
+    const int t = x * q + min(x, rem) + blockIdx.x / 8;
+    const int width = 8 * a.n_blocks, grp = t / width, in = t - grp * width;
+    const int gm = min(a.m_blocks - 8 * grp, 8);
+    mb = 8 * grp + in % gm;
+    nb = in / gm;
+    if (a.n_blocks % 8 == 0) {
+      const int per = a.n_blocks / 8;
+      nb = nb % per * 8 + nb / per;
+    }
+    nb = a.n_blocks - 1 - nb;
+  }
+  const int m0 = mb * kGM, n0 = nb * kGN;
+  const int n64 = a.K / kQkvBK, nk = (n64 + kSub - 1) / kSub;
+  const AppendArgs &ap = a.ap;
+
+  // This wave's loads of a stage: load u = wave + kNW i of its kUnits 1 KB
+  // loads, in each 64-wide K piece those of x (8 rows of 128 bytes each), then
+  // those of W; a wave past the last load repeats it (the same bytes to the
+  // same place), so every wave issues kGPer loads and the waits are exact.
+  // A lane's offset from the tile's first row is 32 bits (kWide: 64).
+  using Off = std::conditional_t<kWide, uint64_t, uint32_t>;
+  const char *xb = (const char *)(a.x + (int64_t)m0 * a.x_stride);
+  const char *wb = (const char *)(a.w + (int64_t)n0 * a.K);
+  Off off[kGPer];
+#pragma unroll
+  for (int i = 0; i < kGPer; i++) {
+    const int c = min(wave + kNW * i, kUnits - 1) % (kXC + kWC);
+    const int r8 = lane >> 3, s = lane & 7;
+    if (c < kXC) {
+      const int r = 8 * c + r8;
+      off[i] = (Off)((int64_t)min(r, a.M - 1 - m0) * a.x_stride + 8 * qkv_slot(r, s)) * 2;
+    } else {
+      const int r = 8 * (c - kXC) + r8;
+      off[i] = (Off)((int64_t)min(r, a.N - 1 - n0) * a.K + 8 * qkv_slot(r, s)) * 2;
+    }
+  }
+  // load i of chunk kc into stage st; K pieces past the last re-read the last one
+  const uint32_t stage_lds = lds_addr(stage);
+  auto dma = [&](int kc, int st, int i) {
+    // the wave's loads split evenly between x and W: which is which is known
+    // when compiling
+    constexpr bool kEven = kSub == 1 && kXC % kNW == 0 && kWC % kNW == 0;
+    const int u = kEven ? wave + kNW * i : min(wave + kNW * i, kUnits - 1);
+    const int sub = kEven ? 0 : u / (kXC + kWC);
+    const bool is_x = kEven ? i < kXC / kNW : u % (kXC + kWC) < kXC;
+    const int64_t kb = (int64_t)min(kc * kSub + sub, n64 - 1) * (kQkvBK * 2);
+    const char *base = (is_x ? xb : wb) + kb;
+    if constexpr (kWide)
+      dma16(base + off[i], &stage[st * kStageElems + u * 512]);
+    else
+      dma16_at(base, off[i], stage_lds + 2 * (st * kStageElems + u * 512));
+  };
+  auto dma_chunk = [&](int kc, int st) {
+#pragma unroll
+    for (int i = 0; i < kGPer; i++)
+      dma(kc, st, i);
   };
 
-  // ---- main loop
-  const int wm = wave % kWM, wn = wave / kWM;
+  Place pl;
+  pl.s_seq = s_place;
+  pl.s_rpos = s_place + Place::kRows;
+  pl.s_len = s_place + 2 * Place::kRows;
+  pl.s_id = s_place + 3 * Place::kRows;
+  pl.s_pos = s_place + 4 * Place::kRows;
+  pl.s_off = s_place + 5 * Place::kRows;
+  pl.s_base = s_base;
+  pl.m0 = m0;
+  pl.wave = wave;
+  pl.prl = 64 * wave + lane;
+  pl.pr = min(m0 + pl.prl, a.M - 1);
+  pl.place = wave < Place::kRows / 64 && ap.kc != nullptr;
+  pl.need_len = ap.seq_lens && (!ap.row_pos || ap.ring > 0);
+
+  const int wm = wave % kWM, wn = (wave / kWM) % kWN, wk = wave / (kWM * kWN);
   f32x4 acc[kRT][4];
 #pragma unroll
   for (int i = 0; i < kRT; i++)
@@ -190,178 +427,187 @@ __global__ __launch_bounds__(64 * kNW) void qkv_append_kernel(QkvArgs a) {
     for (int j = 0; j < 4; j++)
       acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  place_hop1();
+  // operands of one slice, double-buffered: operand q of slice sl of stage st
+  // (W's four, then the row tiles' of x)
+  bf16x8 xo[2][kRT], wo[2][4];
+  auto read = [&](int st, int sl, int q, bf16x8 (&xr)[kRT], bf16x8 (&wr)[4]) {
+    const int k32 = wk + kWK * sl; // slice of the stage
+    const uint16_t *xs = &stage[st * kStageElems + (k32 >> 1) * kSubElems];
+    const uint16_t *ws = xs + kGM * kQkvBK;
+    const int s = 4 * (k32 & 1) + kg;
+    if (q < 4) {
+      const int r = 64 * wn + 16 * q + n;
+      wr[q] = *(const bf16x8 *)&ws[r * kQkvBK + 8 * qkv_slot(r, s)];
+    } else {
+      const int r = 16 * (kRT * wm + q - 4) + n;
+      xr[q - 4] = *(const bf16x8 *)&xs[r * kQkvBK + 8 * qkv_slot(r, s)];
+    }
+  };
+  pl.hop1(ap);
 #pragma unroll
-  for (int p = 0; p < kGStages - 1; p++)
-    dma(p, p);
-  int st = 0;
-  for (int kc = 0; kc < nk; kc++) {
-    // chunk kc landed (only the next kGStages - 2 chunks and the placement
-    // loads issued after chunk kc may still fly); the barrier also frees the
-    // stage of chunk kc - 1 for chunk kc + kGStages - 1
-    wait_vmcnt<(kGStages - 2) * kGPer>();
-    lds_barrier();
-    if (kc == 0)
-      place_hop2(); // hop 1 was issued before chunk 0
-    else if (kc == kGStages - 1)
-      place_hop3(); // hop 2 was issued in iteration 0, before chunk kGStages - 1
-    dma(kc + kGStages - 1, st == 0 ? kGStages - 1 : st - 1);
-    const uint16_t *xs = x_st[st], *ws = w_st[st];
+  for (int p = 0; p < kGStages; p++)
+    dma_chunk(p, p);
+  wait_vmcnt<(kGStages - 1) * kGPer>();
+  lds_barrier();
+  pl.hop2(ap); // hop 1 was issued before chunk 0
 #pragma unroll
-    for (int ks = 0; ks < kGK / 32; ks++) {
-      bf16x8 xo[kRT], wo[4];
+  for (int q = 0; q < 4 + kRT; q++)
+    read(0, 0, q, xo[0], wo[0]);
+  int st = 0; // stage of chunk kc
+  // One chunk, its first slice's operands in buffer b0. Before its last slice's
+  // matrix ops, chunk kc + 1 has landed, every wave has read the whole of chunk
+  // kc (its reads were waited for before the barrier) and chunk kc + kGStages
+  // goes into its stage. The reads of the next slice and those loads are laid
+  // between the row tiles' matrix ops, in this order (the scheduling barriers:
+  // the compiler else moves the reads down to their use and the loads in front
+  // of the matrix ops, and both are waited for).
+  auto chunk = [&](int kc, auto b0c) {
+    constexpr int b0 = decltype(b0c)::value;
+    const int nst = st == kGStages - 1 ? 0 : st + 1;
+#pragma unroll
+    for (int sl = 0; sl < kSl; sl++) {
+      const int cur = (b0 + sl) & 1, nxt = cur ^ 1;
+      const bool last = sl == kSl - 1;
+      if (last) {
+        wait_vmcnt<(kGStages - 2) * kGPer>();
+        lds_barrier();
+        if (kc == kGStages)
+          pl.hop3(ap, a.M); // hop 2 was issued before chunk kGStages's loads
+      }
+      // a K piece past the last adds nothing
+      const bool real = kSub == 1 || kc * kSub + ((wk + kWK * sl) >> 1) < n64;
 #pragma unroll
       for (int i = 0; i < kRT; i++) {
-        const int r = 16 * kRT * wm + 16 * i + n, s = 4 * ks + kg;
-        xo[i] = *(const bf16x8 *)&xs[r * kGK + 8 * (s ^ swz(r))];
-      }
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int r = 64 * wn + 16 * j + n, s = 4 * ks + kg;
-        wo[j] = *(const bf16x8 *)&ws[r * kGK + 8 * (s ^ swz(r))];
+        for (int q = i * (4 + kRT) / kRT; q < (i + 1) * (4 + kRT) / kRT; q++)
+          read(last ? nst : st, last ? 0 : sl + 1, q, xo[nxt], wo[nxt]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (real) {
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            acc[i][j] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(wo[cur][j], xo[cur][i], acc[i][j], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (last) {
+#pragma unroll
+          for (int d = i * kGPer / kRT; d < (i + 1) * kGPer / kRT; d++)
+            dma(kc + kGStages, st, d);
+        }
       }
+    }
+    st = nst;
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  for (int kc = 0; kc < nk; kc += 2 - (kSl + 1) % 2) {
+    chunk(kc, I0{});
+    if constexpr (kSl % 2 == 1) {
+      if (kc + 1 < nk)
+        chunk(kc + 1, I1{});
+    }
+  }
+  wait_vmcnt<0>(); // every load landed, none still writes LDS
+  if (nk <= kGStages) { // a short K left hop 3 for here
+    pl.hop3(ap, a.M);
+    wait_vmcnt<0>();
+  }
+  pl.finish(ap);
+  __syncthreads();
+  if constexpr (kWK > 1) { // the stages are free: the other slices' sums, in wave order
+    f32x4 *red = (f32x4 *)stage + lane;
+    constexpr int kTile = kRT * 4 * 64;
+    if (wk > 0) {
 #pragma unroll
       for (int i = 0; i < kRT; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xo[i], wo[j], acc[i][j], 0, 0, 0);
+          red[(wave - kWM * kWN) * kTile + (4 * i + j) * 64] = acc[i][j];
     }
-    st = st == kGStages - 1 ? 0 : st + 1;
+    __syncthreads();
+    if (wk > 0)
+      return;
+#pragma unroll
+    for (int k = 1; k < kWK; k++)
+#pragma unroll
+      for (int i = 0; i < kRT; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          acc[i][j] += red[(wave + (k - 1) * kWM * kWN) * kTile + (4 * i + j) * 64];
   }
-  wait_vmcnt<0>(); // every load landed, none still writes LDS
-  // a short K (fewer than kGStages chunks) left hop 3 for here
-  if (nk <= kGStages - 1) {
-    place_hop3();
-    wait_vmcnt<0>();
-  }
-  place_finish();
-  __syncthreads();
 
-  // ---- epilogue. acc[i][j][r] is row m0 + 16 kRT wm + 16 i + 4 kg + r,
-  // column n0 + 64 wn + 16 j + n: head hd, dim d = 16 j + n.
   const int hd = (n0 >> 6) + wn;
-  const int c0 = 64 * hd;
-  if (c0 >= a.N)
+  if (64 * hd >= a.N)
     return;
-  float bias[4];
+  f32x4 bias[4];
 #pragma unroll
   for (int j = 0; j < 4; j++)
-    bias[j] = a.bias ? a.bias[c0 + 16 * j + n] : 0.0f;
+    bias[j] = a.bias ? (f32x4) * (const f32x4u *)(a.bias + 64 * hd + 16 * j + 4 * kg)
+                     : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // the wave's staged V rows: its own part of the stages (with kWK > 1 the
+  // part its second slice sums came in)
+  constexpr int kStBytes = kRT * 16 * 128;
+  char *vst = (char *)stage + (wm + kWM * wn) * (kWK > 1 ? 2 : 1) * kStBytes;
 #pragma unroll
   for (int i = 0; i < kRT; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        acc[i][j][r] += bias[j];
-  if (a.out) {
-#pragma unroll
-    for (int i = 0; i < kRT; i++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int m = m0 + 16 * kRT * wm + 16 * i + 4 * kg + r;
-        if (m < a.M) {
-#pragma unroll
-          for (int j = 0; j < 4; j++)
-            a.out[(int64_t)m * a.out_stride + c0 + 16 * j + n] = acc[i][j][r];
-        }
-      }
+    qkv_store_row<kGM>(a, pl, acc[i], bias, hd, 16 * (kRT * wm + i) + n, kg, vst, 16 * i + n);
+  const int gv = hd - ap.n_q_heads - ap.n_kv_heads;
+  if (ap.kc && gv >= 0) {
+    const int row_bytes = ap.v_int8 || ap.kv_fp8 ? 64 : 128;
+    for (int r = 0; r < 16 * kRT; r += 64)
+      qkv_store_values<kGM>(ap, pl, vst + r * row_bytes, 16 * kRT * wm + r,
+                            min(16 * kRT - r, 64), gv, lane);
   }
-  if (!appends || hd < ap.n_q_heads)
-    return;
-  constexpr int D = kHeadDim, HALF = kHeadDim / 2;
-  const bool is_k = hd < ap.n_q_heads + ap.n_kv_heads;
-  const int g = is_k ? hd - ap.n_q_heads : hd - ap.n_q_heads - ap.n_kv_heads;
-#pragma unroll
-  for (int i = 0; i < kRT; i++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int lr = 16 * kRT * wm + 16 * i + 4 * kg + r; // row within the tile
-      const int off = s_off[lr];
-      const int64_t base = s_base[lr] + (int64_t)g * (kBlockTokens * D);
-      const bool st_ok = m0 + lr < a.M && off >= 0;
-      if (is_k) {
-        const int pos = s_pos[lr];
-        float kr[4]; // dims n, 16 + n (first of their pairs), 32 + n, 48 + n
-#pragma unroll
-        for (int j = 0; j < 2; j++) { // dims d = 16 j + n and d + 32
-          const int d = 16 * j + n;
-          const float c = ap.cos_tab[(int64_t)pos * HALF + d];
-          const float s = ap.sin_tab[(int64_t)pos * HALF + d];
-          const float x1 = acc[i][j][r], x2 = acc[i][j + 2][r];
-          kr[j] = rope_first(x1, x2, c, s);
-          kr[j + 2] = rope_second(x1, x2, c, s);
-        }
-        if (ap.kv_fp8) {
-          // e4m3 K: the head's max |k| over its 64 dims (16 lanes), one
-          // scale per token and head, each code stored by its lane
-          float amax = 0.0f;
-#pragma unroll
-          for (int j = 0; j < 4; j++)
-            amax = fmaxf(amax, fabsf(kr[j]));
-#pragma unroll
-          for (int sh = 1; sh < 16; sh <<= 1)
-            amax = fmaxf(amax, __shfl_xor(amax, sh));
-          const float inv = amax > 0.0f ? 448.0f / amax : 0.0f;
-          if (st_ok) {
-            uint8_t *kq = (uint8_t *)ap.kc + base;
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-              kq[k_fp8_offset(off, 16 * j + n)] = (uint8_t)fp8x4(kr[j], 0.0f, 0.0f, 0.0f, inv);
-            if (n == 0)
-              ap.vs[base / 32 + off] = amax / 448.0f;
-          }
-        } else if (st_ok) {
-#pragma unroll
-          for (int j = 0; j < 4; j++)
-            ap.kc[base + k_offset(off, 16 * j + n)] = f32_to_bf16_rne(kr[j]);
-        }
-      } else if (ap.kv_fp8) {
-        // e4m3 V: as the key, codes in the int8 V layout, the scale after
-        // the token's K scale
-        float amax = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          amax = fmaxf(amax, fabsf(acc[i][j][r]));
-#pragma unroll
-        for (int sh = 1; sh < 16; sh <<= 1)
-          amax = fmaxf(amax, __shfl_xor(amax, sh));
-        const float inv = amax > 0.0f ? 448.0f / amax : 0.0f;
-        if (st_ok) {
-          uint8_t *vq = (uint8_t *)ap.vc + base;
-#pragma unroll
-          for (int j = 0; j < 4; j++)
-            vq[v_int8_offset(16 * j + n, off)] = (uint8_t)fp8x4(acc[i][j][r], 0.0f, 0.0f, 0.0f, inv);
-          if (n == 0)
-            ap.vs[base / 32 + kBlockTokens + off] = amax / 448.0f;
-        }
-      } else if (ap.v_int8) {
-        // the head's max |v| over its 64 dims (4 per lane, 16 lanes), then
-        // the reference's rule, getp-csrc/kernels/fast_misc.hpp:74-84
-        float amax = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          amax = fmaxf(amax, fabsf(acc[i][j][r]));
-#pragma unroll
-        for (int sh = 1; sh < 16; sh <<= 1)
-          amax = fmaxf(amax, __shfl_xor(amax, sh));
-        const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
-        if (st_ok) {
-          int8_t *vq = (int8_t *)ap.vc + base;
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const float cq = fminf(fmaxf(rintf(acc[i][j][r] * inv), -127.0f), 127.0f);
-            vq[v_int8_offset(16 * j + n, off)] = (int8_t)cq;
-          }
-          if (n == 0)
-            ap.vs[base / D + off] = amax / 127.0f;
-        }
-      } else if (st_ok) {
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          ap.vc[base + v_offset(off, 16 * j + n)] = f32_to_bf16_rne(acc[i][j][r]);
-      }
-    }
+}
+
+// ---- launch shapes ----------------------------------------------------------------
+
+struct QkvShape {
+  int bm, bn, threads;
+  void (*fn)(QkvArgs);
+};
+
+template <int kGM, int kGN, int kWM, int kWK, int kSub, int kGStages, bool kWide = false>
+static QkvShape shape_of() {
+  return QkvShape{kGM, kGN, 64 * kWM * (kGN / 64) * kWK,
+                  qkv_append_kernel<kGM, kGN, kWM, kWK, kSub, kGStages, kWide>};
+}
+
+// The launch shape for M rows and N columns. Times below: N = 5120, K = 2880,
+// the append included, one MI355X.
+static QkvShape qkv_shape(int M, int N, int64_t x_stride, int K) {
+  auto blocks = [](int64_t n, int b) { return (n + b - 1) / b; };
+  auto tiles = [&](int bm, int bn) { return blocks(M, bm) * blocks(N, bn); };
+  // offsets within a tile beyond 32 bits (a row stride of millions of values)
+  const int64_t x_span = (int64_t)std::min(M, 256) * x_stride * 2;
+  const int64_t w_span = (int64_t)std::min(N, 256) * K * 2;
+  if (x_span > UINT32_MAX || w_span > UINT32_MAX)
+    return shape_of<64, 64, 4, 1, 1, 3, true>();
+  // Few rows: a pass is the chain of its K steps, so each step is wide and its
+  // 32-wide slices are dealt to the waves (16-row tiles, 256-wide steps: 12
+  // steps instead of 45; 24 rows 11.8 us, 32-row tiles 12.3, 64-row ones with
+  // 64-wide steps 16.8). 32-row tiles while every CU gets at most one (64 rows
+  // 12.9 us, 64-row tiles 17.3) or two (128 rows 16.9 against 18.0).
+  if (M <= 32)
+    return shape_of<16, 64, 1, 8, 4, 3>();
+  if (tiles(32, 64) <= 256)
+    return shape_of<32, 64, 2, 4, 2, 4>();
+  if (tiles(32, 64) <= 512)
+    return shape_of<32, 64, 2, 2, 1, 4>();
+  // 64 x 64 tiles while the GPU holds them at up to three per CU (512 rows, 640
+  // tiles: 31.5 us; every larger tile level, 31.6 - 31.8), 128 x 64 ones up to
+  // two per CU (640 rows 32.1 us against 41.2).
+  if (tiles(64, 64) <= 640)
+    return shape_of<64, 64, 4, 1, 1, 3>();
+  if (tiles(128, 64) <= 512)
+    return shape_of<128, 64, 4, 2, 1, 3>();
+  // 128 x 128 tiles (two per CU) take 0.10 - 0.13 us each at any count, 256 x
+  // 256 ones (one per CU) 78 - 85 us a round of 256, the time of some 640 of
+  // the small: 1024 rows 47.0 us against 78, 2048 rows 79.9 against 77.4, 3072
+  // rows 99.3 against 85.5, 9507 rows 302 against 243.
+  if (blocks(tiles(256, 256), 256) * 640 > tiles(128, 128))
+    return shape_of<128, 128, 4, 1, 1, 2>();
+  return shape_of<256, 256, 2, 1, 1, 2>();
 }
 
 } // namespace gkv
@@ -415,12 +661,10 @@ extern "C" int gkv_qkv_append(void *stream, int32_t n_rows, const void *x, int64
   a.M = n_rows;
   a.N = (int)n_cols;
   a.K = hidden;
-  const bool big = n_rows >= kQkvBigRows;
-  const int bm = big ? kQkvBigBM : kQkvBM, bn = big ? kQkvBigBN : kQkvBN;
-  a.m_blocks = (n_rows + bm - 1) / bm;
-  const int n_blocks = (int)((n_cols + bn - 1) / bn);
-  a.xcd_map = n_blocks % 8 == 0;
-  const int64_t grid = (int64_t)a.m_blocks * n_blocks;
+  const QkvShape sh = qkv_shape(n_rows, (int)n_cols, x_stride, hidden);
+  a.m_blocks = (n_rows + sh.bm - 1) / sh.bm;
+  a.n_blocks = (int)((n_cols + sh.bn - 1) / sh.bn);
+  const int64_t grid = (int64_t)a.m_blocks * a.n_blocks;
   if (grid >= INT32_MAX)
     return GKV_ERR_ARG;
   AppendArgs &ap = a.ap;
@@ -447,12 +691,6 @@ extern "C" int gkv_qkv_append(void *stream, int32_t n_rows, const void *x, int64
   ap.v_int8 = cache.v_format == GKV_V_INT8;
   ap.kv_fp8 = cache.v_format == GKV_KV_FP8;
   ap.vs = (float *)cache.v_scale;
-  if (big)
-    hipLaunchKernelGGL(
-        (qkv_append_kernel<kQkvBigBM, kQkvBigBN, kQkvBK, kQkvBigStages, kQkvBigWaves>),
-        dim3((unsigned)grid), dim3(64 * kQkvBigWaves), 0, (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL((qkv_append_kernel<kQkvBM, kQkvBN, kQkvBK, kQkvStages, kQkvWaves>),
-                       dim3((unsigned)grid), dim3(64 * kQkvWaves), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(sh.fn, dim3((unsigned)grid), dim3(sh.threads), 0, (hipStream_t)stream, a);
   return launch_status(__func__);
 }

@@ -307,3 +307,56 @@ def test_bad_block_id_flagged(gkv, cuda):
     poison = np.full_like(res["k1"], np.int16(np.uint16(0x7FC1).view(np.int16)))
     assert np.array_equal(res["k1"], res["k2"])
     assert not np.array_equal(res["k1"], poison)
+
+
+@pytest.mark.parametrize("rows", [1, 17, 32, 33, 96, 97, 192, 193, 512, 513, 768, 769, 1985])
+def test_launch_shapes(oracle, gkv, cuda, rows):
+    """Rows at the edges of the launch shapes of 5120 columns (16-row tiles up
+    to 32 rows, 32-row ones up to 192, 64 x 64 up to 512, 128 x 64 up to 768,
+    then 128 x 128 and 256 x 256), the last row block full or ragged; hidden
+    576 leaves the 256-wide steps of the few-row shape a partial last one."""
+    import torch
+    rng = np.random.default_rng(rows)
+    case = QkvCase(rows, 64, 8, 576, lens=rng.integers(1, 40, rows), v_int8=rows % 3 == 1,
+                   kv_fp8=rows % 3 == 2)
+    res = run(case, gkv, torch, cuda)
+    assert res["err"] == 0
+    check_projection(case, res, oracle, np.unique([0, rows // 2, rows - 1] +
+                                                  list(range(rows // 64 * 64, rows))))
+    check_cache(case, res, oracle)
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+def test_prompt_rows_large_tiles(oracle, gkv, cuda, fmt):
+    """Prompts whose packed rows start at every offset within a 4-token group
+    (values stored four tokens at a time, the others alone) in 256 x 256 tiles."""
+    import torch
+    rng = np.random.default_rng(5 + fmt)
+    prompts = [1, 2, 5] + list(rng.integers(3, 70, 54))
+    case = QkvCase(fmt, 64, 8, 320, prompts=prompts, v_int8=fmt == 1, kv_fp8=fmt == 2)
+    assert case.M > 1792
+    res = run(case, gkv, torch, cuda)
+    assert res["err"] == 0
+    check_projection(case, res, oracle, [0, 777, case.M - 1])
+    check_cache(case, res, oracle)
+
+
+def test_rows_four_gigabytes_apart(gkv, cuda):
+    """A row stride whose byte offsets within a tile pass 32 bits: the same
+    rows as with the tight stride."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    x = torch.empty(2, 128, dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    w = torch.empty(3 * D, 128, dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    far = torch.empty((1 << 31) + 128, dtype=torch.bfloat16, device="cuda")
+    far = far.as_strided((2, 128), (1 << 31, 1))
+    far.copy_(x)
+    out = [torch.empty(2, 3 * D, device="cuda") for _ in range(2)]
+    for xi, o in zip((x, far), out):
+        gkv.qkv_append(xi, w, None, 1, None, None, None, qkv_out=o, n_kv_heads=1)
+    torch.cuda.synchronize()
+    ref = (x.double() @ w.double().t()).cpu().numpy()
+    scale = (x.double().abs() @ w.double().abs().t()).cpu().numpy()
+    for o in out:
+        assert (np.abs(o.cpu().numpy() - ref) <= 2e-5 * scale + 1e-6).all()
