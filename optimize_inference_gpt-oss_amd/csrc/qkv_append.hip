@@ -30,7 +30,7 @@
 //
 // Placement of each row (its sequence, position, slot and block) is loaded by
 // the first waves in three dependent hops of direct-to-LDS loads spread over the
-// first main-loop iterations, so its round trips overlap the loop instead of
+// stages (the largest tile: the first loads), so its round trips overlap them instead of
 // adding to it.
 #include "gkv_device.hpp"
 #include "kv_append.hpp"
@@ -71,65 +71,67 @@ template <int kGM>
 struct QkvPlace {
   static constexpr int kRows = (kGM + 63) / 64 * 64; // 64 per placing wave
   int *s_seq, *s_rpos, *s_len, *s_id; // kRows ints each, 16-byte aligned
-  int *s_pos, *s_off;
-  int64_t *s_base;
-  int m0, wave, prl, pr;
+  int *s_pos, *s_off;                 // the results: position, slot in the block (-1: not stored)
+  int64_t *s_base;                    // and the block's first element
+  int m0, wave;
   bool place, need_len;
-  int p_slot = 0, p_pos = 0;
-  bool p_store = false;
 
-  __device__ __forceinline__ int row_seq_of(const AppendArgs &ap) const {
-    return ap.row_seq ? s_seq[prl] : pr;
+  // The row of this lane within the tile, formed afresh at each use (kept, it
+  // and what is derived from it would hold registers through the main loop).
+  __device__ __forceinline__ int tile_row() const {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
   }
-  __device__ __forceinline__ void hop1(const AppendArgs &ap) {
+  __device__ __forceinline__ int row(int M) const { return min(m0 + tile_row(), M - 1); }
+  __device__ __forceinline__ int row_seq_of(const AppendArgs &ap, int M) const {
+    return ap.row_seq ? s_seq[tile_row()] : row(M);
+  }
+  __device__ __forceinline__ void hop1(const AppendArgs &ap, int M) {
     if (!place)
       return;
     if (ap.row_seq)
-      dma4(ap.row_seq + pr, s_seq + 64 * wave);
+      dma4(ap.row_seq + row(M), s_seq + 64 * wave);
     if (ap.row_pos)
-      dma4(ap.row_pos + pr, s_rpos + 64 * wave);
+      dma4(ap.row_pos + row(M), s_rpos + 64 * wave);
   }
-  __device__ __forceinline__ void hop2(const AppendArgs &ap) { // hop 1 has landed
+  __device__ __forceinline__ void hop2(const AppendArgs &ap, int M) { // hop 1 has landed
     if (!place || !need_len)
       return;
-    dma4(ap.seq_lens + row_seq_of(ap), s_len + 64 * wave);
+    dma4(ap.seq_lens + row_seq_of(ap, M), s_len + 64 * wave);
   }
   __device__ __forceinline__ void hop3(const AppendArgs &ap, int M) { // hop 2 has landed
     if (!place)
       return;
-    const int seq = row_seq_of(ap);
-    const int len = need_len ? s_len[prl] : 0;
-    const int pos = ap.row_pos ? s_rpos[prl] : len - 1;
-    p_pos = pos;
-    p_slot = ap.ring > 0 ? pos % ap.ring : pos;
-    p_store = prl < kGM && m0 + prl < M && pos >= 0;
-    if (p_store && ap.ring > 0 && ap.seq_lens && pos + ap.ring < len)
-      p_store = false; // a later row of this call takes the ring slot
-    const int blk = p_slot / kBlockTokens;
-    if (p_store && blk >= ap.table_stride) {
+    const int r = tile_row();
+    const int seq = row_seq_of(ap, M);
+    const int len = need_len ? s_len[r] : 0;
+    const int pos = ap.row_pos ? s_rpos[r] : len - 1;
+    const int slot = ap.ring > 0 ? pos % ap.ring : pos;
+    bool store = r < kGM && m0 + r < M && pos >= 0;
+    if (store && ap.ring > 0 && ap.seq_lens && pos + ap.ring < len)
+      store = false; // a later row of this call takes the ring slot
+    const int blk = slot / kBlockTokens;
+    if (store && blk >= ap.table_stride) {
       if (ap.dev_err)
         atomicOr(ap.dev_err, GKV_DEVERR_LENGTH);
-      p_store = false;
+      store = false;
     }
+    s_pos[r] = max(pos, 0);
+    s_off[r] = store ? slot % kBlockTokens : -1;
     // rows that are not stored load entry 0 (any valid address)
-    dma4(ap.table + (p_store ? (int64_t)seq * ap.table_stride + blk : 0), s_id + 64 * wave);
+    dma4(ap.table + (store ? (int64_t)seq * ap.table_stride + blk : 0), s_id + 64 * wave);
   }
   __device__ __forceinline__ void finish(const AppendArgs &ap) { // every load has landed
-    if (wave >= kRows / 64)
+    if (!place)
       return;
-    int64_t base = -1;
-    if (place && p_store) {
-      const int id = s_id[prl];
-      if (id < 0 || id >= ap.num_blocks) {
-        if (ap.dev_err)
-          atomicOr(ap.dev_err, GKV_DEVERR_BLOCK_ID);
-      } else {
-        base = (int64_t)id * ap.n_kv_heads * (kBlockTokens * kHeadDim);
-      }
+    const int r = tile_row(), id = s_id[r];
+    s_base[r] = (int64_t)id * ap.n_kv_heads * (kBlockTokens * kHeadDim);
+    if (s_off[r] >= 0 && (id < 0 || id >= ap.num_blocks)) {
+      if (ap.dev_err)
+        atomicOr(ap.dev_err, GKV_DEVERR_BLOCK_ID);
+      s_off[r] = -1;
     }
-    s_pos[prl] = max(p_pos, 0);
-    s_off[prl] = base >= 0 ? p_slot % kBlockTokens : -1;
-    s_base[prl] = base;
   }
 };
 
@@ -369,9 +371,15 @@ __global__ __launch_bounds__(64 * kWM * (kGN / 64) * kWK) void qkv_append_kernel
   using Off = std::conditional_t<kWide, uint64_t, uint32_t>;
   const char *xb = (const char *)(a.x + (int64_t)m0 * a.x_stride);
   const char *wb = (const char *)(a.w + (int64_t)n0 * a.K);
-  Off off[kGPer];
+  // the wave's loads split evenly between x and W: which is which is known when
+  // compiling; and each of W's covers a head's 64 rows (N is whole heads), so
+  // that one offset serves them all
+  constexpr bool kEven = kSub == 1 && kXC % kNW == 0 && kWC % kNW == 0;
+  constexpr bool kOneW = kEven && kNW == 8 && !kWide;
+  constexpr int kOffs = kOneW ? kXC / kNW + 1 : kGPer;
+  Off off[kOffs];
 #pragma unroll
-  for (int i = 0; i < kGPer; i++) {
+  for (int i = 0; i < kOffs; i++) {
     const int c = min(wave + kNW * i, kUnits - 1) % (kXC + kWC);
     const int r8 = lane >> 3, s = lane & 7;
     if (c < kXC) {
@@ -385,18 +393,19 @@ __global__ __launch_bounds__(64 * kWM * (kGN / 64) * kWK) void qkv_append_kernel
   // load i of chunk kc into stage st; K pieces past the last re-read the last one
   const uint32_t stage_lds = lds_addr(stage);
   auto dma = [&](int kc, int st, int i) {
-    // the wave's loads split evenly between x and W: which is which is known
-    // when compiling
-    constexpr bool kEven = kSub == 1 && kXC % kNW == 0 && kWC % kNW == 0;
     const int u = kEven ? wave + kNW * i : min(wave + kNW * i, kUnits - 1);
     const int sub = kEven ? 0 : u / (kXC + kWC);
     const bool is_x = kEven ? i < kXC / kNW : u % (kXC + kWC) < kXC;
     const int64_t kb = (int64_t)min(kc * kSub + sub, n64 - 1) * (kQkvBK * 2);
     const char *base = (is_x ? xb : wb) + kb;
+    const uint32_t dst = stage_lds + 2 * (st * kStageElems + u * 512);
     if constexpr (kWide)
       dma16(base + off[i], &stage[st * kStageElems + u * 512]);
+    else if (kOneW && !is_x) // 64 columns on, or the last 64
+      dma16_at(base + (int64_t)min(64 * (i - kXC / kNW), (a.N - 64 - n0)) * a.K * 2,
+               off[kXC / kNW], dst);
     else
-      dma16_at(base, off[i], stage_lds + 2 * (st * kStageElems + u * 512));
+      dma16_at(base, off[i], dst);
   };
   auto dma_chunk = [&](int kc, int st) {
 #pragma unroll
@@ -414,8 +423,6 @@ __global__ __launch_bounds__(64 * kWM * (kGN / 64) * kWK) void qkv_append_kernel
   pl.s_base = s_base;
   pl.m0 = m0;
   pl.wave = wave;
-  pl.prl = 64 * wave + lane;
-  pl.pr = min(m0 + pl.prl, a.M - 1);
   pl.place = wave < Place::kRows / 64 && ap.kc != nullptr;
   pl.need_len = ap.seq_lens && (!ap.row_pos || ap.ring > 0);
 
@@ -443,13 +450,25 @@ __global__ __launch_bounds__(64 * kWM * (kGN / 64) * kWK) void qkv_append_kernel
       xr[q - 4] = *(const bf16x8 *)&xs[r * kQkvBK + 8 * qkv_slot(r, s)];
     }
   };
-  pl.hop1(ap);
+  pl.hop1(ap, a.M);
+  // The placement's later hops: with 8 row tiles a wave has no registers for
+  // them in the main loop, so hop 1 is waited for behind chunk 0's loads, and
+  // hop 2 goes out before chunk 1 and lands with chunk 0.
+  constexpr bool kEarly = kRT >= 8;
+  if constexpr (kEarly) {
+    dma_chunk(0, 0);
+    wait_vmcnt<kGPer>();
+    pl.hop2(ap, a.M);
+  }
 #pragma unroll
-  for (int p = 0; p < kGStages; p++)
+  for (int p = kEarly ? 1 : 0; p < kGStages; p++)
     dma_chunk(p, p);
   wait_vmcnt<(kGStages - 1) * kGPer>();
   lds_barrier();
-  pl.hop2(ap); // hop 1 was issued before chunk 0
+  if constexpr (kEarly)
+    pl.hop3(ap, a.M);
+  else
+    pl.hop2(ap, a.M); // hop 1 was issued before chunk 0
 #pragma unroll
   for (int q = 0; q < 4 + kRT; q++)
     read(0, 0, q, xo[0], wo[0]);
@@ -471,7 +490,7 @@ __global__ __launch_bounds__(64 * kWM * (kGN / 64) * kWK) void qkv_append_kernel
       if (last) {
         wait_vmcnt<(kGStages - 2) * kGPer>();
         lds_barrier();
-        if (kc == kGStages)
+        if (!kEarly && kc == kGStages)
           pl.hop3(ap, a.M); // hop 2 was issued before chunk kGStages's loads
       }
       // a K piece past the last adds nothing
@@ -508,14 +527,17 @@ __global__ __launch_bounds__(64 * kWM * (kGN / 64) * kWK) void qkv_append_kernel
     }
   }
   wait_vmcnt<0>(); // every load landed, none still writes LDS
-  if (nk <= kGStages) { // a short K left hop 3 for here
+  if (!kEarly && nk <= kGStages) { // a short K left hop 3 for here
     pl.hop3(ap, a.M);
     wait_vmcnt<0>();
   }
   pl.finish(ap);
   __syncthreads();
+  // (the lane's indices formed afresh: kept, they would hold registers through
+  // the main loop)
+  const int elane = pl.tile_row() & 63, en = elane & 15, ekg = elane >> 4;
   if constexpr (kWK > 1) { // the stages are free: the other slices' sums, in wave order
-    f32x4 *red = (f32x4 *)stage + lane;
+    f32x4 *red = (f32x4 *)stage + elane;
     constexpr int kTile = kRT * 4 * 64;
     if (wk > 0) {
 #pragma unroll
@@ -550,13 +572,13 @@ __global__ __launch_bounds__(64 * kWM * (kGN / 64) * kWK) void qkv_append_kernel
   char *vst = (char *)stage + (wm + kWM * wn) * (kWK > 1 ? 2 : 1) * kStBytes;
 #pragma unroll
   for (int i = 0; i < kRT; i++)
-    qkv_store_row<kGM>(a, pl, acc[i], bias, hd, 16 * (kRT * wm + i) + n, kg, vst, 16 * i + n);
+    qkv_store_row<kGM>(a, pl, acc[i], bias, hd, 16 * (kRT * wm + i) + en, ekg, vst, 16 * i + en);
   const int gv = hd - ap.n_q_heads - ap.n_kv_heads;
   if (ap.kc && gv >= 0) {
     const int row_bytes = ap.v_int8 || ap.kv_fp8 ? 64 : 128;
     for (int r = 0; r < 16 * kRT; r += 64)
       qkv_store_values<kGM>(ap, pl, vst + r * row_bytes, 16 * kRT * wm + r,
-                            min(16 * kRT - r, 64), gv, lane);
+                            min(16 * kRT - r, 64), gv, elane);
   }
 }
 
