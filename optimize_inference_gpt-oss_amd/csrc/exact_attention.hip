@@ -14,28 +14,50 @@
 // the 64 output dims, the query heads.
 //
 // Attention: one workgroup per (sequence, kv head, chunk of hc query heads),
-// one wave per query head. The kv head's K rows go through LDS in tiles of 64
-// positions (read once for the hc heads, 65-float rows so that lane t reading
-// row t meets no bank conflict); lane t of wave h scores position t of the
-// tile for head h. The scores stay in LDS, hc x (n + 1) floats (hc is chosen
-// on the host so they fit), through the max, the exponentials, the sum (lane
-// 0, in order), the quotients and the weighted sum of V (lane = output dim),
-// whose rows go through the same LDS tile as K's.
+// `parts` waves per head. Bound by latency: chains whose order is the CPU's (a
+// score's 64 fp64 adds, a head's n adds of the softmax sum, a dim's n FMAs), so
+// each phase runs as many chains side by side as it has and keeps loads out of
+// them:
+//   scores   a wave takes 64 positions, a lane walks one position's K row, 16
+//            dims fetched ahead, with up to eight heads' chains at once on it;
+//   softmax  max, exponentials and quotients over the waves of a head; the
+//            sum in order by one wave per head, its values made fp64 64 at a time;
+//   output   a wave per head, lane = output dim, V rows through a 4-stage LDS
+//            ring that the other waves fill.
+// The scores stay in LDS, hc rows of n + 1 floats (hc is chosen on the host so
+// they fit). Before, K and V went through one LDS tile for one wave per head,
+// and the sum's values were fetched one by one: 32 sequences of 128 .. 2048
+// tokens, 64 / 8 heads, 294 us, now 90 (the longest sequence's scores 35, sum 17,
+// output 35). Contexts of at most kExactShort positions keep that form.
 #include <algorithm>
 
 #include "exact_math.hpp"
 #include "gkv_device.hpp"
+#include "lds_dma.hpp"
 
 namespace gkv {
 
 constexpr int kExactTile = 64;
-constexpr int kExactRow = kHeadDim + 1; // LDS row of a staged K position, in floats
+constexpr int kExactRow = kHeadDim + 1; // LDS row of a staged position (short contexts), in floats
+constexpr int kExactMaxWaves = 16;
+// Contexts of up to this many positions take the one-tile form: there a row per
+// lane, read by every head's waves, costs more than the chains it saves (32
+// sequences on a 128-slot ring: 15.9 us against 19.7; 200 positions level; 600
+// positions, 4 sequences: 68.7 us against 35.4).
+constexpr int kExactShort = 192;
+
+// Four floats at any float's alignment (the fp32 caches' rows).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 struct ExactAttnArgs {
   const float *q;
   int64_t q_stride;
   const float *kc, *vc;
   int slots, n_kv_heads, G, hc, n_chunks, window;
+  int parts;                // waves per head
+  int att_row;              // floats per score row (a multiple of 4)
+  int v_early;              // the V ring has LDS of its own
+  int v_rows;               // V rows per stage of the output's ring (16 per loading wave at most)
   const float *sinks;
   int pos;                  // every row's position (positions == nullptr)
   const int32_t *positions; // device [B], or nullptr
@@ -45,7 +67,260 @@ struct ExactAttnArgs {
   uint32_t *dev_err;
 };
 
-__global__ __launch_bounds__(1024) void attention_exact_kernel(ExactAttnArgs a) {
+// Scores of this lane's position (its K row at kr) for heads h0 .. h0 + NH - 1
+// of the chunk: (float)((sum_i (double)(q_i * k_i)) / sqrt(64)), products rounded
+// to fp32, the sum in order (the division by 8 is exact as a product). The
+// heads' chains run side by side over the row (many: 16 dims fetched ahead).
+// Heads past the last one repeat it (the same value to the same place).
+template <int NH>
+__device__ __forceinline__ void exact_scores(const float *kr, const float *qs, int h0, int hc,
+                                             int j, int n, float *att, int att_row) {
+  double s[NH];
+  const float *q0[NH];
+#pragma unroll
+  for (int hh = 0; hh < NH; hh++) {
+    s[hh] = 0.0;
+    q0[hh] = qs + min(h0 + hh, hc - 1) * kHeadDim;
+  }
+  if constexpr (NH <= 2) { // the whole row at once: one round trip
+    f32x4 k[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+      k[i] = *(const f32x4u *)(kr + 4 * i);
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+#pragma unroll
+      for (int hh = 0; hh < NH; hh++) {
+        const f32x4 q = *(const f32x4 *)&q0[hh][4 * i];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          s[hh] = __dadd_rn(s[hh], (double)__fmul_rn(q[e], k[i][e]));
+      }
+  } else {
+    f32x4 cur[4], nxt[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      cur[i] = *(const f32x4u *)(kr + 4 * i);
+#pragma unroll 1
+    for (int d = 0; d < kHeadDim; d += 16) {
+      const int dn = min(d + 16, kHeadDim - 16); // (the last round re-reads its own)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        nxt[i] = *(const f32x4u *)(kr + dn + 4 * i);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+#pragma unroll
+        for (int hh = 0; hh < NH; hh++) {
+          const f32x4 q = *(const f32x4 *)&q0[hh][d + 4 * i];
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            s[hh] = __dadd_rn(s[hh], (double)__fmul_rn(q[e], cur[i][e]));
+        }
+        __builtin_amdgcn_sched_barrier(0); // (no registers to fetch every query at once)
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        cur[i] = nxt[i];
+    }
+  }
+  if (j < n) {
+#pragma unroll
+    for (int hh = 0; hh < NH; hh++)
+      att[min(h0 + hh, hc - 1) * att_row + j] = (float)__dmul_rn(s[hh], 0.125);
+  }
+}
+
+__global__ __launch_bounds__(64 * kExactMaxWaves) void attention_exact_kernel(ExactAttnArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  __shared__ double s_sum[kExactMaxWaves];
+  __shared__ float s_max[kExactMaxWaves];
+  const int b = blockIdx.x;
+  const int g = blockIdx.y / a.n_chunks;
+  const int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int n_waves = blockDim.x >> 6; // hc * parts
+  const int hc = a.hc;
+  const int hq0 = g * a.G + (blockIdx.y % a.n_chunks) * hc; // the chunk's first query head
+  const int kv_dim = a.n_kv_heads * kHeadDim;
+  float *qs = lds;                  // [hc][64]
+  float *att = qs + hc * kHeadDim;  // [hc][att_row]
+  double *s_dbl = (double *)(att + hc * a.att_row); // [hc][2][64], then the V ring
+
+  const int p = a.positions ? a.positions[b] : a.pos;
+  const int t0 = a.window > 0 ? max(0, p - a.window + 1) : 0;
+  const int n = p - t0 + 1;
+  // a position the cache cannot hold (full layer: p >= slots) or beyond the
+  // host bound: output zeros and the length flag (uniform per workgroup)
+  if (p < 0 || n > a.n_cap || (a.window == 0 && p >= a.slots)) {
+    for (int i = threadIdx.x; i < hc * kHeadDim; i += blockDim.x)
+      a.out[(int64_t)b * a.out_stride + (int64_t)hq0 * kHeadDim + i] = 0.0f;
+    if (threadIdx.x == 0 && a.dev_err)
+      atomicOr(a.dev_err, GKV_DEVERR_LENGTH);
+    return;
+  }
+  // a window layer's cache is a ring of window slots (n <= ring: position j of
+  // the n attended wraps at most once)
+  const int ring = a.window, s0 = ring > 0 ? t0 % ring : 0;
+  auto slot_of = [&](int j) { return ring > 0 && s0 + j >= ring ? s0 + j - ring : s0 + j; };
+  const float *kbase = a.kc + (int64_t)b * a.slots * kv_dim + (int64_t)g * kHeadDim;
+  const float *vbase = a.vc + (int64_t)b * a.slots * kv_dim + (int64_t)g * kHeadDim;
+  // V ring of the output phase (its comment is there); where the LDS holds it
+  // beside the sums' fp64 values, its first stages are fetched from the start.
+  float *ring_v = (float *)(s_dbl + (a.v_early ? 128 * hc : 0));
+  const int R = a.v_rows;
+  const bool split = n_waves > hc;
+  const int n_load = split ? n_waves - hc : n_waves, me = split ? wave - hc : wave;
+  const int per = (R + n_load - 1) / n_load;
+  auto issue = [&](int c) {
+    if (me < 0)
+      return;
+    int r = min(me, R - 1);
+    for (int i = 0; i < per; i++) {
+      dma4(vbase + (int64_t)slot_of(min(c * R + r, n - 1)) * kv_dim + lane,
+           ring_v + ((c & 3) * R + r) * kHeadDim);
+      r = min(r + n_load, R - 1);
+    }
+  };
+  if (a.v_early)
+    for (int c = 0; c < 3; c++)
+      issue(c);
+  for (int i = threadIdx.x; i < hc * kHeadDim; i += blockDim.x)
+    qs[i] = a.q[(int64_t)b * a.q_stride + (int64_t)hq0 * kHeadDim + i];
+  if ((int)threadIdx.x < hc)
+    att[threadIdx.x * a.att_row + n] = a.sinks[hq0 + threadIdx.x];
+  __syncthreads();
+
+  // Items of one 64-position tile and up to 8 heads, fewer heads where there
+  // would be fewer items than waves (a window, a short context).
+  const int tiles = (n + kExactTile - 1) / kExactTile;
+  int hg = 8;
+  while (hg > 1 && tiles * ((hc + hg - 1) / hg) < n_waves)
+    hg >>= 1;
+  const int n_hg = (hc + hg - 1) / hg;
+  for (int it = wave; it < tiles * n_hg; it += n_waves) {
+    const int tile = it / n_hg, h = (it - tile * n_hg) * hg;
+    const int j = tile * kExactTile + lane;
+    const float *kr = kbase + (int64_t)slot_of(min(j, n - 1)) * kv_dim;
+    const int nh = min(hg, hc - h);
+    if (nh > 4)
+      exact_scores<8>(kr, qs, h, hc, j, n, att, a.att_row);
+    else if (nh > 2)
+      exact_scores<4>(kr, qs, h, hc, j, n, att, a.att_row);
+    else if (nh == 2)
+      exact_scores<2>(kr, qs, h, hc, j, n, att, a.att_row);
+    else
+      exact_scores<1>(kr, qs, h, hc, j, n, att, a.att_row);
+  }
+  __syncthreads();
+
+  // softmax over att[0..n] (run.cpp:335-353): the max (exact in any order),
+  // expf((float)((double)x - max)), the fp64 sum in index order, the quotients
+  const int hl = wave % hc, part = wave / hc; // this wave's head and share
+  float *row = att + hl * a.att_row;
+  float m = -INFINITY;
+  for (int j = part * 64 + lane; j <= n; j += 64 * a.parts)
+    m = fmaxf(m, row[j]);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1)
+    m = fmaxf(m, __shfl_xor(m, off));
+  if (lane == 0)
+    s_max[wave] = m;
+  __syncthreads();
+  for (int i = 0; i < a.parts; i++)
+    m = fmaxf(m, s_max[hl + i * hc]);
+  const double md = (double)m;
+  for (int j = part * 64 + lane; j <= n; j += 64 * a.parts)
+    row[j] = expf_cpu_exact((float)__dsub_rn((double)row[j], md));
+  __syncthreads();
+  if (part == 0) {
+    // 64 values at a time become fp64 side by side and come back two per LDS
+    // read, every lane adding them in order: the chain is the additions alone.
+    // (Values past the sink are +0, which changes no sum of non-negatives.)
+    double *sd = s_dbl + hl * 128;
+    auto stage = [&](int c) {
+      const int j = 64 * c + lane;
+      sd[64 * (c & 1) + lane] = j <= n ? (double)row[j] : 0.0;
+    };
+    double s = 0.0;
+    stage(0);
+    for (int c = 0; 64 * c <= n; c++) {
+      stage(c + 1);
+      typedef double f64x2 __attribute__((ext_vector_type(2)));
+      const f64x2 *x = (const f64x2 *)(sd + 64 * (c & 1));
+      for (int k = 0; k < 32 && 64 * c + 2 * k <= n; k += 8) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const f64x2 v = x[k + i];
+          s = __dadd_rn(s, v[0]);
+          s = __dadd_rn(s, v[1]);
+        }
+      }
+    }
+    if (lane == 0)
+      s_sum[hl] = s;
+  }
+  __syncthreads();
+  // The quotients x / sum in fp64: with the correctly rounded reciprocal y, q =
+  // x y and one correction q + y (x - q sum), the remainder exact by FMA, is
+  // the correctly rounded quotient (Markstein, 1990). x in [0, 1] and sum in [1,
+  // n + 1]: nothing over- or underflows; a NaN stays one.
+  const double sum = s_sum[hl], y = __ddiv_rn(1.0, sum);
+  for (int j = part * 64 + lane; j <= n; j += 64 * a.parts) {
+    const double x = (double)row[j], q = __dmul_rn(x, y);
+    row[j] = (float)__fma_rn(__fma_rn(-q, sum, x), y, q);
+  }
+  __syncthreads();
+
+  // out[d] = fma(w_t, v_t[d], out[d]) over t in order: wave h < hc takes head h,
+  // lane = output dim. The other waves (all, if there are no others) bring V
+  // rows into a ring of 4 stages of R rows, row i of
+  // a stage by loader i % n_load; rows past the last position re-read it, and
+  // loaders short of a row repeat their stage's last, so every loader issues
+  // `per` loads a stage and the wait for all but the two younger stages' (or
+  // fewer) is enough.
+  if (!a.v_early)
+    for (int c = 0; c < 3; c++)
+      issue(c);
+  const float *w = att + min(wave, hc - 1) * a.att_row;
+  float acc = 0.0f;
+  for (int c = 0; c * R < n; c++) {
+    if (per >= 16)
+      wait_vmcnt<32>();
+    else if (per >= 8)
+      wait_vmcnt<16>();
+    else if (per >= 4)
+      wait_vmcnt<8>();
+    else if (per >= 2)
+      wait_vmcnt<4>();
+    else
+      wait_vmcnt<2>();
+    lds_barrier(); // stage c is whole; every wave is done with stage c - 1
+    issue(c + 3);
+    if (wave >= hc)
+      continue;
+    const float *v = ring_v + (c & 3) * R * kHeadDim + lane;
+    const int m_t = min(R, n - c * R);
+    int r = 0;
+    for (; r + 16 <= m_t; r += 16) {
+#pragma unroll
+      for (int e = 0; e < 16; e += 4) {
+        const f32x4 x = *(const f32x4 *)&w[c * R + r + e];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          acc = __fmaf_rn(x[i], v[(r + e + i) * kHeadDim], acc);
+      }
+    }
+    for (; r < m_t; r++)
+      acc = __fmaf_rn(w[c * R + r], v[r * kHeadDim], acc);
+  }
+  wait_vmcnt<0>(); // no load may still write into LDS when the workgroup ends
+  if (wave < hc)
+    a.out[(int64_t)b * a.out_stride + (int64_t)(hq0 + wave) * kHeadDim + lane] = acc;
+}
+
+// Short contexts (kExactShort positions): one wave per head, K and V through one
+// LDS tile of 64 positions (65-float rows so that lane t reading row t meets no
+// bank conflict).
+__global__ __launch_bounds__(1024) void attention_exact_short_kernel(ExactAttnArgs a) {
   extern __shared__ float lds[];
   __shared__ double s_sum[16];
   const int b = blockIdx.x;
@@ -256,15 +531,16 @@ extern "C" int gkv_attention_exact(void *stream, int32_t B, int32_t n_q_heads,
   if (B == 0)
     return GKV_OK;
   // positions attended at most, then the most query heads per workgroup whose
-  // score rows fit the LDS next to the K tile and the queries
+  // score rows fit the LDS (kFixed: the part of it that stays free of them, the
+  // limit on the positions of one head)
   const int n_cap = window > 0 ? std::min(p_bound + 1, (int)window) : p_bound + 1;
-  const size_t fixed = (size_t)kExactTile * kExactRow * sizeof(float) + 256; // + s_sum
+  constexpr size_t kFixed = (size_t)kExactTile * (kHeadDim + 1) * sizeof(float) + 256;
   const size_t lim = lds_limit();
   int hc = 0;
   for (int c = G; c >= 1; c--) {
     if (G % c)
       continue;
-    const size_t need = fixed + (size_t)c * (kHeadDim + n_cap + 1) * sizeof(float);
+    const size_t need = kFixed + (size_t)c * (kHeadDim + n_cap + 1) * sizeof(float);
     if (need <= lim) {
       hc = c;
       break;
@@ -272,7 +548,6 @@ extern "C" int gkv_attention_exact(void *stream, int32_t B, int32_t n_q_heads,
   }
   if (hc == 0)
     return GKV_ERR_CAPACITY;
-  const size_t lds = fixed - 256 + (size_t)hc * (kHeadDim + n_cap + 1) * sizeof(float);
   ExactAttnArgs a{};
   a.q = q;
   a.q_stride = q_stride;
@@ -291,11 +566,38 @@ extern "C" int gkv_attention_exact(void *stream, int32_t B, int32_t n_q_heads,
   a.out = out;
   a.out_stride = out_stride;
   a.dev_err = dev_err;
+  size_t lds;
+  int threads;
+  void (*fn)(ExactAttnArgs);
+  if (n_cap <= kExactShort) {
+    lds = kFixed - 256 + (size_t)hc * (kHeadDim + n_cap + 1) * sizeof(float);
+    threads = 64 * hc;
+    fn = attention_exact_short_kernel;
+  } else {
+    a.att_row = (n_cap + 1 + 3) / 4 * 4;
+    // waves: a whole number per head, at most one per head and 64-position tile
+    const int tiles = (n_cap + kExactTile - 1) / kExactTile;
+    a.parts = std::max(1, std::min(kExactMaxWaves / hc, tiles));
+    // The V ring: 4 stages of 64 rows where the LDS has room
+    // and the loading waves need at most 16 loads each, else of 16 rows, which
+    // kFixed always holds (then in the place of the sums' fp64 values).
+    const size_t rows_bytes = (size_t)hc * (kHeadDim + a.att_row) * sizeof(float);
+    const size_t dbl_bytes = (size_t)hc * 128 * sizeof(double);
+    auto ring_bytes = [](int rows) { return (size_t)4 * rows * kHeadDim * sizeof(float); };
+    const int waves = hc * a.parts, n_load = waves > hc ? waves - hc : waves;
+    const size_t room = lim - 256 - rows_bytes; // (256: the static arrays)
+    a.v_rows = n_load >= 4 && ring_bytes(64) + dbl_bytes <= room ? 64 : 16;
+    a.v_early = ring_bytes(a.v_rows) + dbl_bytes <= room;
+    lds = rows_bytes + (a.v_early ? ring_bytes(a.v_rows) + dbl_bytes
+                                  : std::max(ring_bytes(a.v_rows), dbl_bytes));
+    threads = 64 * waves;
+    fn = attention_exact_kernel;
+  }
   if (lds > 64 * 1024 &&
-      hipFuncSetAttribute((const void *)attention_exact_kernel,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+      hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)lds) != hipSuccess)
     return hip_status(hipGetLastError(), "attention_exact_kernel (LDS size)");
-  hipLaunchKernelGGL(attention_exact_kernel, dim3(B, n_kv_heads * a.n_chunks), dim3(64 * hc),
-                     lds, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(fn, dim3(B, n_kv_heads * a.n_chunks), dim3(threads), lds,
+                     (hipStream_t)stream, a);
   return launch_status("attention_exact_kernel");
 }

@@ -113,6 +113,12 @@ def _attention_case(seed, B, Hq, Hkv, lens_lo, lens_hi, window=0, slots=None):
     ("long", 2, 16, 2, 9000, 12000, 0),          # score rows past a workgroup's LDS for 8 heads
     ("group16", 3, 32, 2, 1, 3000, 0),           # 16 query heads per kv head (1024 threads)
     ("group1", 3, 4, 4, 1, 700, 64),             # one query head per kv head, a 64-slot ring
+    ("short_form_edge", 3, 16, 2, 192, 192, 0),  # the longest context of the one-tile form
+    ("long_form_edge", 4, 16, 2, 1, 193, 0),     # the first bound of the other, short rows too
+    ("ring256", 4, 12, 2, 200, 900, 256),        # 6 heads a group, rings that wrap
+    ("tiles", 3, 3, 1, 255, 257, 0),             # 64-position tiles full, one short, one over
+    ("group16_wide", 2, 16, 1, 2100, 2300, 0),   # 16 heads at once, 16-row V stages
+    ("lds_full", 1, 8, 1, 4400, 4400, 0),        # the V ring in the sums' place
 ])
 def test_attention_exact_bit_exact(gkv, cuda, name, B, Hq, Hkv, lo, hi, window):
     import torch
