@@ -63,6 +63,12 @@ __device__ __forceinline__ uint32_t fp8x4(float x0, float x1, float x2, float x3
   return (uint32_t)w;
 }
 
+// Eight fp32 values rounded to bf16 as one 16-byte piece, element 0 first.
+__device__ __forceinline__ u32x4 round8(const float *f) {
+  return u32x4{f32x2_to_bf16_rne(f[0], f[1]), f32x2_to_bf16_rne(f[2], f[3]),
+               f32x2_to_bf16_rne(f[4], f[5]), f32x2_to_bf16_rne(f[6], f[7])};
+}
+
 // Eight bf16 (bits) as one 16-byte piece, element 0 first.
 __device__ __forceinline__ u32x4 pack8(const uint16_t *h) {
   return u32x4{h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16),
@@ -79,17 +85,14 @@ __device__ __forceinline__ void append_keys(const AppendArgs &a, int r, int g, i
   constexpr int D = kHeadDim, HALF = kHeadDim / 2;
   const int kv_dim = a.n_kv_heads * D;
   float f1[8], f2[8];
-  uint16_t o1[8], o2[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     const float a1 = x1[i / 4][i % 4], a2 = x2[i / 4][i % 4];
     const float cc = c[i / 4][i % 4], ss = s[i / 4][i % 4];
     f1[i] = rope_first(a1, a2, cc, ss);
     f2[i] = rope_second(a1, a2, cc, ss);
-    o1[i] = f32_to_bf16_rne(f1[i]);
-    o2[i] = f32_to_bf16_rne(f2[i]);
   }
-  const u32x4 p1 = pack8(o1), p2 = pack8(o2);
+  const u32x4 p1 = round8(f1), p2 = round8(f2);
   if (store && a.kv_fp8) {
     // e4m3 K: the head's max |k| over its 4 lanes, then one scale per
     // token and head; the lane's 16 codes are one 16-byte piece
@@ -126,18 +129,19 @@ __device__ __forceinline__ void append_values(const AppendArgs &a, int r, int g,
                                               int off, uint16_t *v_stage) {
   constexpr int D = kHeadDim;
   const int kv_dim = a.n_kv_heads * D;
-  uint16_t h[16];
+  float f[16];
 #pragma unroll
   for (int i = 0; i < 16; i++)
-    h[i] = f32_to_bf16_rne(x[i / 4][i % 4]);
+    f[i] = x[i / 4][i % 4];
+  const u32x4 lo = round8(f), hi = round8(f + 8);
   if (a.v_pack) {
     uint16_t *vpk = a.v_pack + (int64_t)r * kv_dim + g * D + 16 * q;
-    *(u32x4 *)vpk = pack8(h);
-    *(u32x4 *)(vpk + 8) = pack8(h + 8);
+    *(u32x4 *)vpk = lo;
+    *(u32x4 *)(vpk + 8) = hi;
   }
   if (v_stage && !a.v_int8 && !a.kv_fp8) {
-    *(u32x4 *)(v_stage + g * D + 16 * q) = pack8(h);
-    *(u32x4 *)(v_stage + g * D + 16 * q + 8) = pack8(h + 8);
+    *(u32x4 *)(v_stage + g * D + 16 * q) = lo;
+    *(u32x4 *)(v_stage + g * D + 16 * q + 8) = hi;
     return;
   }
   if (!store)
@@ -185,7 +189,7 @@ __device__ __forceinline__ void append_values(const AppendArgs &a, int r, int g,
     uint16_t *vd = a.vc + vbase + (int64_t)g * (kBlockTokens * D);
 #pragma unroll
     for (int i = 0; i < 16; i++)
-      vd[v_offset(off, 16 * q + i)] = h[i];
+      vd[v_offset(off, 16 * q + i)] = (uint16_t)((i < 8 ? lo : hi)[i % 8 / 2] >> (16 * (i & 1)));
   }
 }
 

@@ -231,8 +231,7 @@ __device__ __forceinline__ void qkv_store_row(const QkvArgs &a, const QkvPlace<k
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int d = 16 * j + 4 * kg;
-    const u32x2 w{f32_to_bf16_rne(y[j][0]) | ((uint32_t)f32_to_bf16_rne(y[j][1]) << 16),
-                  f32_to_bf16_rne(y[j][2]) | ((uint32_t)f32_to_bf16_rne(y[j][3]) << 16)};
+    const u32x2 w{f32x2_to_bf16_rne(y[j][0], y[j][1]), f32x2_to_bf16_rne(y[j][2], y[j][3])};
     if (!is_k && quant)
       *(uint32_t *)(vst + v_stage_code(vr, d)) = code[j];
     else if (!is_k)

@@ -271,3 +271,28 @@ def test_prefill_sweep(oracle, gkv, cuda, seed):
     if p["rot"]:
         res["q"] = case.q_rot  # the append wrote no rotated Q
     check(case, res, rtol=RTOL + (2.0 ** -8 if p["bf16"] else 0.0))
+
+
+def test_append_rounds_every_class_of_float(gkv, cuda):
+    """Values of random bit patterns (NaNs, infinities, subnormals, ties among
+    them) as the append packs them: round to nearest even, NaN quiet with the
+    high payload bits kept."""
+    import torch
+    rng = np.random.default_rng(3)
+    n, Hq, Hkv = 2048, 8, 8
+    qkv = rng.standard_normal((n, (Hq + 2 * Hkv) * D)).astype(np.float32)
+    u = rng.integers(0, 1 << 32, (n, Hkv * D), dtype=np.uint64).astype(np.uint32)
+    u[::2, ::3] = (u[::2, ::3] & 0xFFFF0000) | 0x8000   # ties
+    u[::5, ::7] = (u[::5, ::7] & 0x807FFFFF)             # subnormals and zeros
+    u[::5, 1::7] |= 0x7F800000                           # infinities and NaNs
+    qkv.view(np.uint32)[:, (Hq + Hkv) * D:] = u
+    cos, sin = gkv.rope_table(1)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)  # noqa: E731
+    vp = torch.zeros(n, Hkv * D, dtype=torch.int16, device=cuda)
+    kp = torch.zeros_like(vp)
+    gkv.kv_append(d(qkv), Hq, d(cos), d(sin), d(np.zeros(n, np.int32)),
+                  gkv.CacheView(n_kv_heads=Hkv), k_pack=kp, v_pack=vp)
+    torch.cuda.synchronize()
+    nan = (u & 0x7FFFFFFF) > 0x7F800000
+    want = np.where(nan, (u >> 16) | 0x40, (u.astype(np.uint64) + 0x7FFF + ((u >> 16) & 1)) >> 16)
+    assert np.array_equal(vp.cpu().numpy().view(np.uint16), want.astype(np.uint16))
