@@ -25,8 +25,8 @@
 //   A 32-key step uses two 16-key score tiles; lane (kg, n) holds keys
 //   4kg..4kg+3 of each, which are its P^T operand slots; the V^T operand is
 //   the same 8 keys of one dim, read from V stored transposed in LDS.
-// Online softmax in the log2 domain (scale 1/8 * log2 e folded into Q), lazy
-// rescale by threshold 8 (tested on the fp16 weights), the running max seeded
+// Online softmax in the log2 domain (scale 1/8 * log2 e in the exponent's FMA),
+// lazy rescale (tested on the sums of the fp16 weights), the running max seeded
 // with the sink, and the sink added in the final normalisation, as in the
 // decode kernel. The row sums are fp32 sums of the same fp16 weights.
 //
@@ -49,6 +49,15 @@
 // stays in rows. The V of tile t + 1 is turned into V^T [64 dims][64 keys + 8 pad]
 // fp16 after tile t is computed, into the other of two V^T buffers: two
 // barriers per tile, and a tile's loads have two tiles' compute to land in.
+//
+// What bounds it: at short prompts the round trips at a workgroup's start and
+// end, at long ones the vector instructions of the softmax (16 exponentials a
+// lane and 32-key step, about 70 other) beside 24 matrix ops. So the scale
+// stands in the exponent's FMA, the rescale test is one compare of the row sum,
+// the query is split into its pieces two values at a time, and a quantized V's
+// mask and power of two go into its scales: 8 chunks of 100 .. 700 tokens after
+// 1536 cached ones, int8 V, 251 -> 237 us; 64 prompts of 64 .. 512 tokens 228
+// -> 222 us (full layer), 189 -> 185 us (window).
 #include "gkv_device.hpp"
 #include "lds_dma.hpp"
 
@@ -62,8 +71,10 @@ constexpr int kQBlock = 32;         // query positions per workgroup
 constexpr int kKTile = 64;          // keys per LDS tile
 constexpr int kVRow = kKTile + 8;   // fp16 per V^T row in LDS
 constexpr float kVScale = 0x1p-10f; // V is staged as fp16 of v * kVScale
+constexpr float kQScale = 0.125f * kLog2e; // 1/sqrt(64); exp -> exp2 (on the scores)
 constexpr int kStages = 3;          // K/V tile pipeline depth (tiles held in LDS)
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 struct PrefillArgs {
   const int32_t *cu;
@@ -298,8 +309,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW >= 8
         const uint16_t *blk = vs + (r0 >> 4) * 1024;
         const float *scl = (const float *)(blk + 512) + (VF == 2 ? kBlockTokens : 0);
         const int t0 = r0 & 15;
-        const bool keep0 = kt0 + r0 <= p_last, keep1 = kt0 + r1 <= p_last;
-        const float s0 = scl[t0], s1 = scl[t0 + 1];
+        // (the power of two and the mask go into the scales: the products are
+        // the same bits)
+        const float s0 = kt0 + r0 <= p_last ? scl[t0] * kVScale : 0.0f;
+        const float s1 = kt0 + r1 <= p_last ? scl[t0 + 1] * kVScale : 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           const int d = 4 * pd + j;
@@ -309,15 +322,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW >= 8
           float v0, v1;
           if (VF == 2) {
             const f32x2 f = __builtin_amdgcn_cvt_pk_f32_fp8((int)c2, false); // bytes 0, 1
-            v0 = f[0];
-            v1 = f[1];
+            v0 = kt0 + r0 <= p_last ? f[0] : 0.0f; // (an unwritten slot may hold the NaN code)
+            v1 = kt0 + r1 <= p_last ? f[1] : 0.0f;
           } else {
             v0 = (float)(int8_t)(c2 & 0xffu);
             v1 = (float)(int8_t)(c2 >> 8);
           }
-          const float x0 = keep0 ? v0 * s0 : 0.0f;
-          const float x1 = keep1 ? v1 * s1 : 0.0f;
-          hp[j] = f32_half(x0) | (f32_half(x1) << 16);
+          const f16x2 h{(_Float16)(v0 * s0), (_Float16)(v1 * s1)};
+          hp[j] = __builtin_bit_cast(uint32_t, h);
         }
       } else {
         uint32_t pair[4]; // bf16 bits
@@ -494,24 +506,31 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW >= 8
         }
 #pragma unroll
         for (int i = 0; i < 8; i++)
-          ph[c][i] = (_Float16)__builtin_amdgcn_exp2f(sc[i] - m_run[c]);
-        // Lazy rescale: the reference max moves only when a weight exceeds 2^8
-        // (a score more than 8 above it; an fp16 weight of inf included). The
-        // test runs on the fp16 weights with packed max; it needs no cross-lane
-        // max (m_run is the same in the 4 lanes of a column), only the rescale,
-        // which then recomputes the weights.
-        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-        f16x2 w2 = __builtin_elementwise_max(
-            __builtin_elementwise_max(f16x2{ph[c][0], ph[c][1]}, f16x2{ph[c][2], ph[c][3]}),
-            __builtin_elementwise_max(f16x2{ph[c][4], ph[c][5]}, f16x2{ph[c][6], ph[c][7]}));
-        if (__any(__builtin_elementwise_max(w2[0], w2[1]) > (_Float16)256.0f)) {
+          ph[c][i] = (_Float16)__builtin_amdgcn_exp2f(fmaf(sc[i], kQScale, -m_run[c]));
+        // the row sum of the same fp16 weights the output uses (fp32 sums)
+        auto row_sum = [&]() {
+          float t = 0.0f;
+#pragma unroll
+          for (int i = 0; i < 8; i += 2)
+            t = __builtin_amdgcn_fdot2(f16x2{ph[c][i], ph[c][i + 1]},
+                                       f16x2{(_Float16)1.0f, (_Float16)1.0f}, t, false);
+          return t;
+        };
+        float step_sum = row_sum();
+        // Lazy rescale: the reference max moves only when the step's weights sum
+        // to more than 2^8 in some lane (so whenever one of them exceeds that,
+        // an fp16 weight of inf included; a rescale is never wrong), or to a NaN
+        // (the weight of a masked key while the max is a sink of -inf). The test
+        // needs no cross-lane max (m_run is the same in the 4 lanes of a
+        // column), only the rescale, which then recomputes the weights.
+        if (__any(!(step_sum <= 256.0f))) {
           float mx = sc[0];
 #pragma unroll
           for (int i = 1; i < 8; i++)
             mx = fmaxf(mx, sc[i]);
           mx = fmaxf(mx, __shfl_xor(mx, 16));
           mx = fmaxf(mx, __shfl_xor(mx, 32));
-          const float m_new = fmaxf(m_run[c], mx);
+          const float m_new = fmaxf(m_run[c], mx * kQScale);
           const float alpha = __builtin_amdgcn_exp2f(m_run[c] - m_new);
           m_run[c] = m_new;
           lsum[c] *= alpha;
@@ -520,13 +539,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW >= 8
             o[c][nn] *= alpha;
 #pragma unroll
           for (int i = 0; i < 8; i++)
-            ph[c][i] = (_Float16)__builtin_amdgcn_exp2f(sc[i] - m_run[c]);
+            ph[c][i] = (_Float16)__builtin_amdgcn_exp2f(fmaf(sc[i], kQScale, -m_run[c]));
+          step_sum = row_sum();
         }
-        // the row sum of the same fp16 weights the output uses (fp32 sums)
-#pragma unroll
-        for (int i = 0; i < 8; i += 2)
-          lsum[c] = __builtin_amdgcn_fdot2(f16x2{ph[c][i], ph[c][i + 1]},
-                                           f16x2{(_Float16)1.0f, (_Float16)1.0f}, lsum[c], false);
+        lsum[c] += step_sum;
       }
 #pragma unroll
       for (int nn = 0; nn < 4; nn++) {
@@ -553,33 +569,36 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW >= 8
   wait_vmcnt<2 * (8 / NW)>();
   lds_barrier();
   {
-    const float qscale = 0.125f * kLog2e; // 1/sqrt(64); exp -> exp2
+    // rotated (one uniform branch), then split into bf16 high and low pieces two
+    // at a time; the scale goes onto the scores, where it costs nothing
 #pragma unroll
     for (int c = 0; c < 2; c++) {
-      f32x4 cr[2] = {}, sr[2] = {};
       if (rot) {
         const float *cp = ang + (16 * c + n) * (D / 2) + 8 * kg;
-        cr[0] = *(const f32x4 *)cp;
-        cr[1] = *(const f32x4 *)(cp + 4);
-        sr[0] = *(const f32x4 *)(cp + 1024);
-        sr[1] = *(const f32x4 *)(cp + 1028);
-      }
-      float qv[2][8];
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const float x1 = qr[c][j / 4][j % 4], x2 = qr[c][2 + j / 4][j % 4];
-        qv[0][j] = rot ? rope_first(x1, x2, cr[j / 4][j % 4], sr[j / 4][j % 4]) : x1;
-        qv[1][j] = rot ? rope_second(x1, x2, cr[j / 4][j % 4], sr[j / 4][j % 4]) : x2;
+        for (int j4 = 0; j4 < 2; j4++) {
+          const f32x4 cr = *(const f32x4 *)(cp + 4 * j4), sr = *(const f32x4 *)(cp + 1024 + 4 * j4);
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const float x1 = qr[c][j4][j], x2 = qr[c][2 + j4][j];
+            qr[c][j4][j] = rope_first(x1, x2, cr[j], sr[j]);
+            qr[c][2 + j4][j] = rope_second(x1, x2, cr[j], sr[j]);
+          }
+        }
       }
 #pragma unroll
       for (int dh = 0; dh < 2; dh++) {
+        u32x4 hi, lo;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-          const float x = qv[dh][j] * qscale;
-          const __bf16 hi = (__bf16)x;
-          qhi[c][dh][j] = hi;
-          qlo[c][dh][j] = (__bf16)(x - (float)hi);
+        for (int j = 0; j < 4; j++) { // dims 2 j, 2 j + 1 of the lane's 8
+          const f32x2 x{qr[c][2 * dh + j / 2][2 * (j % 2)], qr[c][2 * dh + j / 2][2 * (j % 2) + 1]};
+          hi[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2));
+          const f32x2 l{x[0] - __uint_as_float(hi[j] << 16),
+                        x[1] - __uint_as_float(hi[j] & 0xffff0000u)};
+          lo[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(l, bf16x2));
         }
+        qhi[c][dh] = __builtin_bit_cast(bf16x8, hi);
+        qlo[c][dh] = __builtin_bit_cast(bf16x8, lo);
       }
     }
   }

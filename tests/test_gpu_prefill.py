@@ -273,6 +273,16 @@ def test_prefill_sweep(oracle, gkv, cuda, seed):
     check(case, res, rtol=RTOL + (2.0 ** -8 if p["bf16"] else 0.0))
 
 
+def test_sinks_of_minus_infinity_and_large_scores(oracle, gkv, cuda):
+    """Heads whose sink carries no weight (the running max starts at -inf, so the
+    first step's weights overflow and its masked keys' are NaN until the rescale),
+    beside scores of tens of units that rescale again and again."""
+    import torch
+    case = PrefillCase(oracle, 41, [1, 31, 33, 64, 65, 200, 330], 64, 8, scale=2.0)
+    case.sinks[::3] = -np.inf
+    check(case, run_gpu(case, gkv, torch, cuda))
+
+
 def test_append_rounds_every_class_of_float(gkv, cuda):
     """Values of random bit patterns (NaNs, infinities, subnormals, ties among
     them) as the append packs them: round to nearest even, NaN quiet with the
