@@ -27,7 +27,7 @@
 // The scores stay in LDS, hc rows of n + 1 floats (hc is chosen on the host so
 // they fit). Before, K and V went through one LDS tile for one wave per head,
 // and the sum's values were fetched one by one: 32 sequences of 128 .. 2048
-// tokens, 64 / 8 heads, 294 us, now 90 (the longest sequence's scores 35, sum 17,
+// tokens, 64 / 8 heads, 294 us, now 90 - 95 (the longest sequence's scores 35, sum 17,
 // output 35). Contexts of at most kExactShort positions keep that form.
 #include <algorithm>
 
