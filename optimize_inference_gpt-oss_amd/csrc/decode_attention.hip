@@ -1553,7 +1553,9 @@ __device__ __forceinline__ void combine_head_wide(const DecodeArgs &a, int4 rec,
     for (int i = 0; i < 4; i++)
       if (ok[i])
         Mn = fmaxf(Mn, m[i]);
-    const float c0 = __builtin_amdgcn_exp2f(M - Mn);
+    // (both maxima are -inf after a sink of -inf and ranges without tokens only:
+    // nothing summed yet, and -inf - -inf would be a NaN)
+    const float c0 = __builtin_amdgcn_exp2f(M == Mn ? 0.0f : M - Mn);
     M = Mn;
     Ls *= c0;
     o0 *= c0;

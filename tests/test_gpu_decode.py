@@ -220,6 +220,19 @@ def test_few_sequences_in_more_ranges_than_steps(gkv, cuda, torch_mod, lens):
     check_case(case, run_gpu(case, gkv, torch_mod, cuda))
 
 
+@pytest.mark.parametrize("lens, split_tokens", [
+    ([40], 0), ([500], 0), ([4095], 0), ([1500, 0, 2, 700], 0), ([20000, 3], 0),
+    ([0, 31, 127, 159, 1023, 2431], 32)])
+def test_combine_with_sinks_of_no_weight(gkv, cuda, torch_mod, lens, split_tokens):
+    # sinks of -inf, and of the lowest float (-inf once in log2 units): with the
+    # balanced split a wave of the combine meets only ranges without tokens
+    # first, so that its running max is the sink alone
+    case = DecodeCase(len(lens), 64, 8, np.array(lens, np.int32), window=0, seed=37, scale=0.7)
+    case.sinks[::3] = -np.inf
+    case.sinks[1::3] = np.finfo(np.float32).min
+    check_case(case, run_gpu(case, gkv, torch_mod, cuda, split_tokens=split_tokens))
+
+
 def test_rotated_q_path_and_bf16_output(gkv, cuda, torch_mod):
     L = np.array([3, 200, 900, 64], np.int32)
     case = DecodeCase(len(L), 64, 8, L, window=0, scale=0.5, seed=66)
