@@ -50,7 +50,11 @@ __device__ __forceinline__ void dma16(const void *src, void *l_base) {
 }
 
 // dma16 with a wave-uniform base address (held in SGPRs) and a 32-bit byte
-// offset per lane: no 64-bit address per lane is formed or kept.
+// offset per lane: no 64-bit address per lane is formed or kept. The base's
+// halves may come from v_readfirstlane right before the asm, and a memory
+// instruction may read an SGPR five wait states after a vector instruction
+// wrote it at the earliest. The compiler waits in front of its own
+// instructions only, so the asm brings all five (the moves count one each).
 __device__ __forceinline__ void dma16_s(const void *base, uint32_t byte_off, void *l_base) {
   const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)l_base);
   const uint64_t b = (uint64_t)(uintptr_t)base;
@@ -62,7 +66,7 @@ __device__ __forceinline__ void dma16_s(const void *base, uint32_t byte_off, voi
   uint32_t saved;
   asm volatile("s_mov_b32 %0, m0\n\t"
                "s_mov_b32 m0, %3\n\t"
-               "s_nop 0\n\t"
+               "s_nop 2\n\t"
                "global_load_lds_dwordx4 %1, %2\n\t"
                "s_mov_b32 m0, %0"
                : "=&s"(saved)
@@ -84,7 +88,7 @@ __device__ __forceinline__ void dma16_at(const void *base, uint32_t byte_off, ui
   const uint64_t sb = ((uint64_t)hi << 32) | lo;
   const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane(lds);
   asm volatile("s_mov_b32 m0, %2\n\t"
-               "s_nop 0\n\t"
+               "s_nop 3\n\t"
                "global_load_lds_dwordx4 %0, %1"
                :
                : "v"(byte_off), "s"(sb), "s"(m)

@@ -103,6 +103,39 @@ def test_direct_to_lds_scalar_bases_are_not_sign_extended(tmp_path):
     assert n_loads > 0
 
 
+@pytest.mark.timeout(600)
+@pytest.mark.parametrize("src", ["qkv_append", "prefill_attention"])
+def test_direct_to_lds_scalar_bases_are_old_enough(tmp_path, src):
+    """A memory instruction may read an SGPR five wait states after a vector
+    instruction wrote it, at the earliest (the hardware does not check). The
+    compiler inserts them in front of its own instructions, but not of one in
+    inline asm: the asm of the loads with a scalar base has to bring them, for
+    a base that v_readfirstlane wrote right before it."""
+    n_loads = 0
+    lines = []
+    for l in device_asm(tmp_path, src).splitlines():
+        l = l.split(";")[0].strip()
+        if not l or l.startswith(".") or l.endswith(":"):
+            continue
+        lines.append(l)
+        m = re.match(r"global_load_lds_\w+ v\d+, s\[(\d+):(\d+)\]", l)
+        if not m:
+            continue
+        n_loads += 1
+        base = {"s" + m.group(1), "s" + m.group(2)}
+        states = 0
+        for d in reversed(lines[:-1]):
+            if states >= 5:
+                break
+            w = re.match(r"v_\w+ (s\d+|s\[\d+:\d+\]),", d)
+            if w:
+                regs = {w.group(1)} if "[" not in w.group(1) else _pair_regs(d)
+                assert not regs & base, f"{src}: {l} {states} wait states after {d}"
+            nop = re.match(r"s_nop (\d+)", d)
+            states += int(nop.group(1)) + 1 if nop else 1
+    assert n_loads > 0
+
+
 def _pair_regs(line):
     m = re.match(r"(s_|v_)\w+ s\[(\d+):(\d+)\]", line.strip())
     return {"s" + str(i) for i in range(int(m.group(2)), int(m.group(3)) + 1)}
