@@ -28,7 +28,7 @@
 // they fit). Before, K and V went through one LDS tile for one wave per head,
 // and the sum's values were fetched one by one: 32 sequences of 128 .. 2048
 // tokens, 64 / 8 heads, 294 us, now 90 - 95 (the longest sequence's scores 35, sum 17,
-// output 35). Contexts of at most kExactShort positions keep that form.
+// output 35). Short contexts, and middling ones of many sequences, keep that form.
 #include <algorithm>
 
 #include "exact_math.hpp"
@@ -45,6 +45,16 @@ constexpr int kExactMaxWaves = 16;
 // sequences on a 128-slot ring: 15.9 us against 19.7; 200 positions level; 600
 // positions, 4 sequences: 68.7 us against 35.4).
 constexpr int kExactShort = 192;
+// With more workgroups than a round of the long form holds (one per CU, its V
+// ring and fp64 values taking 82 KB and more of LDS; a CU holds 3 or 4 of the
+// one-tile form, and those overlap each other's chains) the line lies higher,
+// for three or more heads a workgroup (with fewer the long form is ahead
+// throughout). 64 / 8 heads, long against one-tile form, us: 64 sequences, 300
+// positions each 51 / 57; 96 of 300 each 75 / 67; 512 of 200 each 327 / 228, of 500
+// each 505 / 511, of 1 .. 500 435 / 362, of 1 .. 600 471 / 425, of 1 .. 700 512 / 577; 192
+// of 1 .. 500 174 / 160, of 1 .. 600 186 / 204.
+constexpr int kExactShortMany = 512, kExactShortVeryMany = 640;
+constexpr int64_t kExactMany = 2 * 256, kExactVeryMany = 8 * 256; // workgroups, 256 CUs
 
 // Four floats at any float's alignment (the fp32 caches' rows).
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -317,7 +327,7 @@ __global__ __launch_bounds__(64 * kExactMaxWaves) void attention_exact_kernel(Ex
     a.out[(int64_t)b * a.out_stride + (int64_t)(hq0 + wave) * kHeadDim + lane] = acc;
 }
 
-// Short contexts (kExactShort positions): one wave per head, K and V through one
+// Short contexts (the rule is at kExactShort): one wave per head, K and V through one
 // LDS tile of 64 positions (65-float rows so that lane t reading row t meets no
 // bank conflict).
 __global__ __launch_bounds__(1024) void attention_exact_short_kernel(ExactAttnArgs a) {
@@ -569,7 +579,11 @@ extern "C" int gkv_attention_exact(void *stream, int32_t B, int32_t n_q_heads,
   size_t lds;
   int threads;
   void (*fn)(ExactAttnArgs);
-  if (n_cap <= kExactShort) {
+  const int64_t wgs = (int64_t)B * n_kv_heads * a.n_chunks;
+  const int short_cap = hc < 3 || wgs <= kExactMany ? kExactShort
+                        : wgs <= kExactVeryMany     ? kExactShortMany
+                                                    : kExactShortVeryMany;
+  if (n_cap <= short_cap) {
     lds = kFixed - 256 + (size_t)hc * (kHeadDim + n_cap + 1) * sizeof(float);
     threads = 64 * hc;
     fn = attention_exact_short_kernel;

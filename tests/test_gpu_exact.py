@@ -119,6 +119,11 @@ def _attention_case(seed, B, Hq, Hkv, lens_lo, lens_hi, window=0, slots=None):
     ("tiles", 3, 3, 1, 255, 257, 0),             # 64-position tiles full, one short, one over
     ("group16_wide", 2, 16, 1, 2100, 2300, 0),   # 16 heads at once, 16-row V stages
     ("lds_full", 1, 8, 1, 4400, 4400, 0),        # the V ring in the sums' place
+    ("many", 65, 64, 8, 1, 512, 0),              # just over 512 workgroups: the one-tile form
+    ("many_long", 65, 24, 8, 500, 513, 0),       # ... up to 512 positions, 3 heads a group
+    ("very_many", 257, 32, 8, 1, 640, 0),        # over 2048 workgroups: up to 640 positions
+    ("very_many_long", 257, 24, 8, 1, 641, 0),   # one more: the long form
+    ("many_two_heads", 65, 16, 8, 1, 300, 0),    # two heads a group: the long form
 ])
 def test_attention_exact_bit_exact(gkv, cuda, name, B, Hq, Hkv, lo, hi, window):
     import torch
