@@ -76,8 +76,7 @@ __device__ __forceinline__ void dma16_s(const void *base, uint32_t byte_off, voi
 
 // dma16_s in a loop whose LDS and global addresses are kept as numbers: the
 // LDS byte address of the wave's 1 KB (the low half of a generic pointer into
-// LDS is its LDS address) and the base both wave-uniform. M0 is declared
-// overwritten instead of saved, so the load is three instructions.
+// LDS is its LDS address) and the base both wave-uniform.
 __device__ __forceinline__ uint32_t lds_addr(const void *p) {
   return (uint32_t)(uintptr_t)(lds_ptr)p;
 }
@@ -87,12 +86,15 @@ __device__ __forceinline__ void dma16_at(const void *base, uint32_t byte_off, ui
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
   const uint64_t sb = ((uint64_t)hi << 32) | lo;
   const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane(lds);
-  asm volatile("s_mov_b32 m0, %2\n\t"
-               "s_nop 3\n\t"
-               "global_load_lds_dwordx4 %0, %1"
-               :
+  uint32_t saved;
+  asm volatile("s_mov_b32 %0, m0\n\t"
+               "s_mov_b32 m0, %3\n\t"
+               "s_nop 2\n\t"
+               "global_load_lds_dwordx4 %1, %2\n\t"
+               "s_mov_b32 m0, %0" // (M0 is reserved: no clobber may name it)
+               : "=&s"(saved)
                : "v"(byte_off), "s"(sb), "s"(m)
-               : "memory", "m0");
+               : "memory");
 }
 
 // 4 bytes per lane straight into LDS: lane l's dword lands at l_base + 4 l.
