@@ -615,10 +615,14 @@ static QkvShape qkv_shape(int M, int N, int64_t x_stride, int K) {
     return shape_of<32, 64, 2, 4, 2, 4>();
   if (tiles(32, 64) <= 512)
     return shape_of<32, 64, 2, 2, 1, 4>();
-  // 64 x 64 tiles while the GPU holds them at up to three per CU (512 rows, 640
-  // tiles: 31.5 us; every larger tile level, 31.6 - 31.8), 128 x 64 ones up to
-  // two per CU (640 rows 32.1 us against 41.2).
-  if (tiles(64, 64) <= 640)
+  // 64 x 64 tiles up to two per CU, and where a third one goes to a good part of
+  // the CUs (512 rows, 640 tiles: 29.9 us, 128 x 64 ones 30.7); with a third on
+  // few CUs only 128 x 64 ones are ahead (416 rows, 560 tiles: 30.1 against 29.3; N
+  // = 2560, 800 rows, 520 tiles: 30.9 against 28.1), and they are beyond 640 tiles
+  // (540 rows, 720 tiles: 34.8 against 29.1), up to two of them per CU (640 rows
+  // 32.1 us against 41.2).
+  const int64_t t64 = tiles(64, 64);
+  if (t64 <= 512 || (t64 > 576 && t64 <= 640))
     return shape_of<64, 64, 4, 1, 1, 3>();
   if (tiles(128, 64) <= 512)
     return shape_of<128, 64, 4, 2, 1, 3>();

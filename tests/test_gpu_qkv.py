@@ -326,6 +326,22 @@ def test_launch_shapes(oracle, gkv, cuda, rows):
     check_cache(case, res, oracle)
 
 
+@pytest.mark.parametrize("rows, heads", [(384, (64, 8)), (385, (64, 8)), (448, (64, 8)),
+                                         (449, (64, 8)), (800, (32, 4)), (927, (32, 4))])
+def test_launch_shapes_of_two_tiles_per_cu(oracle, gkv, cuda, rows, heads):
+    """Rows around 512 and 576 tiles of 64 x 64 (two per CU, and a third on few of
+    them), where the row tiles change from 64 to 128 and back, on 80 and 40
+    column blocks."""
+    import torch
+    rng = np.random.default_rng(rows)
+    case = QkvCase(rows, heads[0], heads[1], 128, lens=rng.integers(1, 40, rows))
+    res = run(case, gkv, torch, cuda)
+    assert res["err"] == 0
+    check_projection(case, res, oracle, np.unique([0, rows // 2] +
+                                                  list(range(rows // 128 * 128, rows))))
+    check_cache(case, res, oracle)
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2])
 def test_prompt_rows_large_tiles(oracle, gkv, cuda, fmt):
     """Prompts whose packed rows start at every offset within a 4-token group
