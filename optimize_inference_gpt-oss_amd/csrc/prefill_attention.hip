@@ -531,7 +531,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW >= 8
           mx = fmaxf(mx, __shfl_xor(mx, 16));
           mx = fmaxf(mx, __shfl_xor(mx, 32));
           const float m_new = fmaxf(m_run[c], mx * kQScale);
-          const float alpha = __builtin_amdgcn_exp2f(m_run[c] - m_new);
+          // -inf still: a sink of -inf and every key so far masked (a window's
+          // later queries in the oldest step). The weights of -inf are then
+          // taken against 0, since -inf - -inf would be a NaN.
+          const float m_ref = m_new == -INFINITY ? 0.0f : m_new;
+          const float alpha = __builtin_amdgcn_exp2f(m_run[c] - m_ref);
           m_run[c] = m_new;
           lsum[c] *= alpha;
 #pragma unroll
@@ -539,7 +543,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW >= 8
             o[c][nn] *= alpha;
 #pragma unroll
           for (int i = 0; i < 8; i++)
-            ph[c][i] = (_Float16)__builtin_amdgcn_exp2f(fmaf(sc[i], kQScale, -m_run[c]));
+            ph[c][i] = (_Float16)__builtin_amdgcn_exp2f(fmaf(sc[i], kQScale, -m_ref));
           step_sum = row_sum();
         }
         lsum[c] += step_sum;

@@ -283,6 +283,18 @@ def test_sinks_of_minus_infinity_and_large_scores(oracle, gkv, cuda):
     check(case, run_gpu(case, gkv, torch, cuda))
 
 
+@pytest.mark.parametrize("window", [32, 128])
+def test_sinks_of_minus_infinity_on_a_window_layer(oracle, gkv, cuda, window):
+    """The oldest 32-key step of a window is wholly masked for the last queries of
+    a block: with a sink of -inf (or of the lowest float, -inf in log2 units)
+    their running max is still -inf after it."""
+    import torch
+    case = PrefillCase(oracle, 43, [1, 33, 160, 161, 200, 330], 64, 8, window=window, scale=2.0)
+    case.sinks[::3] = -np.inf
+    case.sinks[1::3] = np.finfo(np.float32).min
+    check(case, run_gpu(case, gkv, torch, cuda))
+
+
 def test_append_rounds_every_class_of_float(gkv, cuda):
     """Values of random bit patterns (NaNs, infinities, subnormals, ties among
     them) as the append packs them: round to nearest even, NaN quiet with the

@@ -217,6 +217,27 @@ def test_two_chunks_ring_layer(oracle, gkv, cuda, fmt, window):
 
 
 @pytest.mark.parametrize("fmt", ["bf16", "int8", "fp8"])
+def test_ring_layer_with_sinks_of_minus_infinity(oracle, gkv, cuda, fmt):
+    """A block's later queries see nothing of the window's oldest step, cached or
+    packed: with a sink of -inf their running max is still -inf after it."""
+    import torch
+    c = Chunked(torch, gkv, oracle, [400, 260], [256, 128], window=128, seed=15, fmt=fmt)
+    c.sinks[::3] = -np.inf
+    c.sinks_d = c.t(c.sinks)
+    c.reference()
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    try:
+        c.append(1, err)
+        kp, vp = c.packed(2)
+        got, rows = c.prefill(2, err, k=kp, v=vp)
+        assert np.isfinite(got).all()
+        c.check(got, rows, "chunk 2", n_cached=c.C)
+        assert int(err.item()) == 0
+    finally:
+        c.pool.close()
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "int8", "fp8"])
 @pytest.mark.parametrize("Hq,Hkv", [(8, 2), (8, 4), (8, 8), (12, 2)])
 def test_group_sizes(oracle, gkv, cuda, Hq, Hkv, fmt):
     """Groups of 4, 2, 1 and 6 query heads per kv head (the 4-, 2- and 1-wave
