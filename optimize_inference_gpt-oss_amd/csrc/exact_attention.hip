@@ -53,8 +53,15 @@ constexpr int kExactShort = 192;
 // positions each 51 / 57; 96 of 300 each 75 / 67; 512 of 200 each 327 / 228, of 500
 // each 505 / 511, of 1 .. 500 435 / 362, of 1 .. 600 471 / 425, of 1 .. 700 512 / 577; 192
 // of 1 .. 500 174 / 160, of 1 .. 600 186 / 204.
+// In the second round of the long form (257 .. 512 workgroups) it lies at 256 for
+// five or more heads a workgroup: 8 heads, 264 workgroups of 256 each 46.1 / 42 - 46,
+// 384 of 1 .. 224 44.6 / 33, 512 of 200 each 43.8 / 41, of 1 .. 256 48.2 / 43, of 1 .. 300
+// level. And at 320 for 9 to 15 heads, which leave the long form idle waves (one a
+// head): 512 of 10 heads, 300 each 65.3 / 60 - 62, of 1 .. 400 level; 16 heads, 300 each,
+// level.
+constexpr int kExactShortTwo = 256, kExactShortTwoOdd = 320;
 constexpr int kExactShortMany = 512, kExactShortVeryMany = 640;
-constexpr int64_t kExactMany = 2 * 256, kExactVeryMany = 8 * 256; // workgroups, 256 CUs
+constexpr int64_t kExactTwo = 256, kExactMany = 2 * 256, kExactVeryMany = 8 * 256; // workgroups, 256 CUs
 
 // Four floats at any float's alignment (the fp32 caches' rows).
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -580,9 +587,11 @@ extern "C" int gkv_attention_exact(void *stream, int32_t B, int32_t n_q_heads,
   int threads;
   void (*fn)(ExactAttnArgs);
   const int64_t wgs = (int64_t)B * n_kv_heads * a.n_chunks;
-  const int short_cap = hc < 3 || wgs <= kExactMany ? kExactShort
-                        : wgs <= kExactVeryMany     ? kExactShortMany
-                                                    : kExactShortVeryMany;
+  int short_cap = kExactShort;
+  if (wgs > kExactMany && hc >= 3)
+    short_cap = wgs <= kExactVeryMany ? kExactShortMany : kExactShortVeryMany;
+  else if (wgs > kExactTwo && wgs <= kExactMany && hc >= 5)
+    short_cap = hc > kExactMaxWaves / 2 && hc < kExactMaxWaves ? kExactShortTwoOdd : kExactShortTwo;
   if (n_cap <= short_cap) {
     lds = kFixed - 256 + (size_t)hc * (kHeadDim + n_cap + 1) * sizeof(float);
     threads = 64 * hc;

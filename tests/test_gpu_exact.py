@@ -125,6 +125,11 @@ def _attention_case(seed, B, Hq, Hkv, lens_lo, lens_hi, window=0, slots=None):
     ("very_many", 257, 32, 8, 1, 640, 0),        # over 2048 workgroups: up to 640 positions
     ("very_many_long", 257, 24, 8, 1, 641, 0),   # one more: the long form
     ("many_two_heads", 65, 16, 8, 1, 300, 0),    # two heads a group: the long form
+    ("second_round", 33, 64, 8, 1, 256, 0),      # just over 256 workgroups: one-tile up to 256
+    ("second_round_long", 33, 40, 8, 1, 257, 0),  # one position more, 5 heads: the long form
+    ("second_round_few", 33, 32, 8, 200, 256, 0),  # 4 heads a group: the long form
+    ("second_round_odd", 257, 10, 1, 1, 320, 0),   # 10 heads, no idle waves: one-tile up to 320
+    ("second_round_odd_long", 257, 9, 1, 300, 321, 0),
 ])
 def test_attention_exact_bit_exact(gkv, cuda, name, B, Hq, Hkv, lo, hi, window):
     import torch
