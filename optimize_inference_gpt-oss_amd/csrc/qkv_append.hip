@@ -626,11 +626,15 @@ static QkvShape qkv_shape(int M, int N, int64_t x_stride, int K) {
     return shape_of<64, 64, 4, 1, 1, 3>();
   if (tiles(128, 64) <= 512)
     return shape_of<128, 64, 4, 2, 1, 3>();
-  // 128 x 128 tiles (two per CU) take 0.10 - 0.13 us each at any count, 256 x
-  // 256 ones (one per CU) 78 - 85 us a round of 256, the time of some 640 of
-  // the small: 1024 rows 47.0 us against 78, 2048 rows 79.9 against 77.4, 3072
-  // rows 99.3 against 85.5, 9507 rows 302 against 243.
-  if (blocks(tiles(256, 256), 256) * 640 > tiles(128, 128))
+  // 128 x 128 tiles while the GPU holds them at two per CU, then 256 x 256 ones
+  // (one per CU, rounds of 256, 67 - 78 us each): N = 2560, 3072 rows 48 us against 69,
+  // 3328 rows 79.6 against 69, 6400 rows 108 against 82. A second or third round of
+  // the large tiles pays from some 1420 and 2130 small ones on: N = 2560, 8192
+  // rows (1280) 124.6 against 133.8, 8960 rows (1400) 136.5 against 139.6, 9216 rows
+  // (1440) 146.1 against 140.9; N = 5120, 4352 rows (1360) 129.9 against 140, 4864 rows
+  // (1520) 160 against 141, 6656 rows (2080) level, 7424 rows (2320) 217 against 209.
+  const int64_t t128 = tiles(128, 128), rounds = blocks(tiles(256, 256), 256);
+  if (t128 <= (rounds > 1 ? rounds * 710 : 512))
     return shape_of<128, 128, 4, 1, 1, 2>();
   return shape_of<256, 256, 2, 1, 1, 2>();
 }

@@ -342,6 +342,23 @@ def test_launch_shapes_of_two_tiles_per_cu(oracle, gkv, cuda, rows, heads):
     check_cache(case, res, oracle)
 
 
+@pytest.mark.parametrize("rows, heads", [(1535, (64, 8)), (1537, (64, 8)), (9087, (32, 4)),
+                                         (9089, (32, 4))])
+def test_launch_shapes_of_many_rows(oracle, gkv, cuda, rows, heads):
+    """Rows around the changes from 128 x 128 to 256 x 256 tiles: past 480 of the small
+    ones (the next row block makes 520), and past 1420 against two rounds of the
+    large ones; the last row block one row short, and of one row."""
+    import torch
+    rng = np.random.default_rng(rows)
+    case = QkvCase(rows, heads[0], heads[1], 64, prompts=[500] * (rows // 500) + [rows % 500])
+    assert case.M == rows
+    res = run(case, gkv, torch, cuda)
+    assert res["err"] == 0
+    check_projection(case, res, oracle, np.unique(list(rng.integers(0, rows, 20)) +
+                                                  list(range(rows // 256 * 256, rows, 5))))
+    check_cache(case, res, oracle)
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2])
 def test_prompt_rows_large_tiles(oracle, gkv, cuda, fmt):
     """Prompts whose packed rows start at every offset within a 4-token group
