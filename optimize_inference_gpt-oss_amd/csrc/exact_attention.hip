@@ -28,7 +28,8 @@
 // they fit). Before, K and V went through one LDS tile for one wave per head,
 // and the sum's values were fetched one by one: 32 sequences of 128 .. 2048
 // tokens, 64 / 8 heads, 294 us, now 90 - 95 (the longest sequence's scores 35, sum 17,
-// output 35). Short contexts, and middling ones of many sequences, keep that form.
+// output 35). Short contexts keep that one-tile form: a kernel of its own where
+// the host bound is short, a branch where only a row's own context is.
 #include <algorithm>
 
 #include "exact_math.hpp"
@@ -45,23 +46,20 @@ constexpr int kExactMaxWaves = 16;
 // sequences on a 128-slot ring: 15.9 us against 19.7; 200 positions level; 600
 // positions, 4 sequences: 68.7 us against 35.4).
 constexpr int kExactShort = 192;
-// With more workgroups than a round of the long form holds (one per CU, its V
-// ring and fp64 values taking 82 KB and more of LDS; a CU holds 3 or 4 of the
-// one-tile form, and those overlap each other's chains) the line lies higher,
-// for three or more heads a workgroup (with fewer the long form is ahead
-// throughout). 64 / 8 heads, long against one-tile form, us: 64 sequences, 300
-// positions each 51 / 57; 96 of 300 each 75 / 67; 512 of 200 each 327 / 228, of 500
-// each 505 / 511, of 1 .. 500 435 / 362, of 1 .. 600 471 / 425, of 1 .. 700 512 / 577; 192
-// of 1 .. 500 174 / 160, of 1 .. 600 186 / 204.
-// In the second round of the long form (257 .. 512 workgroups) it lies at 256 for
-// five or more heads a workgroup: 8 heads, 264 workgroups of 256 each 46.1 / 42 - 46,
-// 384 of 1 .. 224 44.6 / 33, 512 of 200 each 43.8 / 41, of 1 .. 256 48.2 / 43, of 1 .. 300
-// level. And at 320 for 9 to 15 heads, which leave the long form idle waves (one a
-// head): 512 of 10 heads, 300 each 65.3 / 60 - 62, of 1 .. 400 level; 16 heads, 300 each,
-// level.
-constexpr int kExactShortTwo = 256, kExactShortTwoOdd = 320;
-constexpr int kExactShortMany = 512, kExactShortVeryMany = 640;
-constexpr int64_t kExactTwo = 256, kExactMany = 2 * 256, kExactVeryMany = 8 * 256; // workgroups, 256 CUs
+// Where one workgroup per CU does not hold the call (kExactTwo workgroups, 256
+// CUs) and two fit a CU's LDS, the long form runs with 64 registers and a smaller
+// V ring, two workgroups of 16 waves to a CU, or (past kExactFour) up to four of
+// 8: their chains overlap each other's. 8 heads a workgroup, us, one-tile form / one
+// to a CU / so: 512 workgroups of 1 .. 40 positions under a bound of 1024 12.5 / 24.3 / 12.0,
+// of 1 .. 1000 161 / 88.8 / 94.5 (384), 1024 of 1 .. 500 under 1500 161 / 128 / 105, 4096 of
+// 1 .. 40 under 1024 57 / 167 / 57, of 1 .. 500 under 1500 565 / 452 / 333.
+// The one-tile form, of which a CU holds four (8 heads), stays ahead further up
+// while that leaves it fewer rounds: to 256 positions with 257 .. 512 workgroups of
+// five or more heads (384 of 1 .. 224 34.6 against 37.3, 512 of 200 each 40 - 42 against 38),
+// to 300 with 513 .. 1024 of 5 to 8 (1024 of 200 each 58.5 against 69.5, 768 of 1 .. 300
+// 58.1 against 69.7, 1024 of 300 level).
+constexpr int kExactShortTwo = 256, kExactShortFour = 300;
+constexpr int64_t kExactTwo = 256, kExactMany = 2 * 256, kExactFour = 4 * 256;
 
 // Four floats at any float's alignment (the fp32 caches' rows).
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -75,6 +73,7 @@ struct ExactAttnArgs {
   int att_row;              // floats per score row (a multiple of 4)
   int v_early;              // the V ring has LDS of its own
   int v_rows;               // V rows per stage of the output's ring (16 per loading wave at most)
+  int one_tile_n;           // rows of at most this many positions take the one-tile form
   const float *sinks;
   int pos;                  // every row's position (positions == nullptr)
   const int32_t *positions; // device [B], or nullptr
@@ -87,9 +86,10 @@ struct ExactAttnArgs {
 // Scores of this lane's position (its K row at kr) for heads h0 .. h0 + NH - 1
 // of the chunk: (float)((sum_i (double)(q_i * k_i)) / sqrt(64)), products rounded
 // to fp32, the sum in order (the division by 8 is exact as a product). The
-// heads' chains run side by side over the row (many: 16 dims fetched ahead).
+// heads' chains run side by side over the row (kWhole: fetched at once, else 16 dims
+// ahead).
 // Heads past the last one repeat it (the same value to the same place).
-template <int NH>
+template <int NH, bool kWhole>
 __device__ __forceinline__ void exact_scores(const float *kr, const float *qs, int h0, int hc,
                                              int j, int n, float *att, int att_row) {
   double s[NH];
@@ -99,7 +99,7 @@ __device__ __forceinline__ void exact_scores(const float *kr, const float *qs, i
     s[hh] = 0.0;
     q0[hh] = qs + min(h0 + hh, hc - 1) * kHeadDim;
   }
-  if constexpr (NH <= 2) { // the whole row at once: one round trip
+  if constexpr (kWhole) { // the whole row at once: one round trip
     f32x4 k[16];
 #pragma unroll
     for (int i = 0; i < 16; i++)
@@ -147,7 +147,135 @@ __device__ __forceinline__ void exact_scores(const float *kr, const float *qs, i
   }
 }
 
-__global__ __launch_bounds__(64 * kExactMaxWaves) void attention_exact_kernel(ExactAttnArgs a) {
+// The one-tile form: a wave per head (waves past the hc heads only load; kAll:
+// there are none), K and V through one LDS tile of 64 positions (65-float rows so
+// that lane t reading row t meets no bank conflict).
+template <bool kAll>
+__device__ __forceinline__ void exact_one_tile(const ExactAttnArgs &a, float *lds, double *s_sum,
+                                               int b, int g, int hq0, int t0, int n) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const bool head = kAll || wave < a.hc;
+  const int hw = kAll ? wave : min(wave, a.hc - 1), h = hq0 + hw;
+  const int kv_dim = a.n_kv_heads * kHeadDim;
+  float *kt = lds;                                   // [64][65]
+  float *qs = kt + kExactTile * kExactRow;           // [hc][64]
+  float *att = qs + a.hc * kHeadDim + hw * (n + 1); // this head's scores
+  const int ring = a.window; // a window layer's cache is a ring of window slots
+  const float *kbase = a.kc + (int64_t)b * a.slots * kv_dim + (int64_t)g * kHeadDim;
+  const float *vbase = a.vc + (int64_t)b * a.slots * kv_dim + (int64_t)g * kHeadDim;
+  if (head)
+    qs[hw * kHeadDim + lane] = a.q[(int64_t)b * a.q_stride + (int64_t)h * kHeadDim + lane];
+
+  // scores: (float)((sum_i (double)(q_i * k_i)) / 8), products rounded to fp32
+  const double scale = (double)__fsqrt_rn((float)kHeadDim);
+  for (int tile = 0; tile < n; tile += kExactTile) {
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < kExactTile * kHeadDim; idx += blockDim.x) {
+      const int r = idx >> 6, c = idx & 63, j = tile + r;
+      if (j < n) {
+        const int t = t0 + j;
+        const int slot = ring > 0 ? t % ring : t;
+        kt[r * kExactRow + c] = kbase[(int64_t)slot * kv_dim + c];
+      }
+    }
+    __syncthreads();
+    const int j = tile + lane;
+    if (head && j < n) {
+      double s = 0.0;
+      for (int i = 0; i < kHeadDim; i++)
+        s = __dadd_rn(s, (double)__fmul_rn(qs[hw * kHeadDim + i], kt[lane * kExactRow + i]));
+      att[j] = (float)__ddiv_rn(s, scale);
+    }
+  }
+  if (head && lane == 0)
+    att[n] = a.sinks[h];
+  __syncthreads();
+
+  // softmax over att[0..n] (run.cpp:335-353): the max (exact in any order),
+  // expf((float)((double)x - max)), the fp64 sum in index order, the quotients
+  if (head) {
+    float m = -INFINITY;
+    for (int j = lane; j <= n; j += 64)
+      m = fmaxf(m, att[j]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+      m = fmaxf(m, __shfl_xor(m, off));
+    const double md = (double)m;
+    for (int j = lane; j <= n; j += 64)
+      att[j] = expf_cpu_exact((float)__dsub_rn((double)att[j], md));
+  }
+  __syncthreads();
+  if (head && lane == 0) {
+    double s = 0.0;
+#pragma unroll 8
+    for (int j = 0; j <= n; j++)
+      s = __dadd_rn(s, (double)att[j]);
+    s_sum[hw] = s;
+  }
+  __syncthreads();
+  if (head) {
+    const double sum = s_sum[hw];
+    for (int j = lane; j <= n; j += 64)
+      att[j] = (float)__ddiv_rn((double)att[j], sum);
+  }
+  __syncthreads();
+
+  // out[d] = fma(w_t, v_t[d], out[d]) over t in order; the V rows go through
+  // the K tile's LDS, 64 positions at a time, read once for the hc heads
+  float acc = 0.0f;
+  for (int tile = 0; tile < n; tile += kExactTile) {
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < kExactTile * kHeadDim; idx += blockDim.x) {
+      const int r = idx >> 6, c = idx & 63, j = tile + r;
+      if (j < n) {
+        const int t = t0 + j;
+        const int slot = ring > 0 ? t % ring : t;
+        kt[r * kExactRow + c] = vbase[(int64_t)slot * kv_dim + c];
+      }
+    }
+    __syncthreads();
+    if (head) {
+      const int m_t = min(kExactTile, n - tile);
+      for (int r = 0; r < m_t; r++)
+        acc = __fmaf_rn(att[tile + r], kt[r * kExactRow + lane], acc);
+    }
+  }
+  if (head)
+    a.out[(int64_t)b * a.out_stride + (int64_t)h * kHeadDim + lane] = acc;
+}
+
+// A workgroup's row: positions t0 .. t0 + n - 1, or false after zeros and the
+// length flag for a position the cache cannot hold (full layer: p >= slots) or
+// beyond the host bound (uniform per workgroup).
+__device__ __forceinline__ bool exact_row(const ExactAttnArgs &a, int b, int hq0, int &t0, int &n) {
+  const int p = a.positions ? a.positions[b] : a.pos;
+  t0 = a.window > 0 ? max(0, p - a.window + 1) : 0;
+  n = p - t0 + 1;
+  if (p >= 0 && n <= a.n_cap && (a.window > 0 || p < a.slots))
+    return true;
+  for (int i = threadIdx.x; i < a.hc * kHeadDim; i += blockDim.x)
+    a.out[(int64_t)b * a.out_stride + (int64_t)hq0 * kHeadDim + i] = 0.0f;
+  if (threadIdx.x == 0 && a.dev_err)
+    atomicOr(a.dev_err, GKV_DEVERR_LENGTH);
+  return false;
+}
+
+__global__ __launch_bounds__(64 * kExactMaxWaves) void attention_exact_short_kernel(ExactAttnArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  __shared__ double s_sum[kExactMaxWaves];
+  const int b = blockIdx.x, g = blockIdx.y / a.n_chunks;
+  const int hq0 = g * a.G + (blockIdx.y % a.n_chunks) * a.hc; // the chunk's first query head
+  int t0, n;
+  if (exact_row(a, b, hq0, t0, n))
+    exact_one_tile<true>(a, lds, s_sum, b, g, hq0, t0, n);
+}
+
+// kLite: 64 registers, so that the waves of two workgroups of 16 or four of 8 fit a
+// CU (the rule is in the host code).
+template <bool kLite>
+__global__ __launch_bounds__(64 * kExactMaxWaves)
+__attribute__((amdgpu_waves_per_eu(kLite ? 8 : 4)))
+void attention_exact_kernel(ExactAttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   __shared__ double s_sum[kExactMaxWaves];
   __shared__ float s_max[kExactMaxWaves];
@@ -162,16 +290,11 @@ __global__ __launch_bounds__(64 * kExactMaxWaves) void attention_exact_kernel(Ex
   float *att = qs + hc * kHeadDim;  // [hc][att_row]
   double *s_dbl = (double *)(att + hc * a.att_row); // [hc][2][64], then the V ring
 
-  const int p = a.positions ? a.positions[b] : a.pos;
-  const int t0 = a.window > 0 ? max(0, p - a.window + 1) : 0;
-  const int n = p - t0 + 1;
-  // a position the cache cannot hold (full layer: p >= slots) or beyond the
-  // host bound: output zeros and the length flag (uniform per workgroup)
-  if (p < 0 || n > a.n_cap || (a.window == 0 && p >= a.slots)) {
-    for (int i = threadIdx.x; i < hc * kHeadDim; i += blockDim.x)
-      a.out[(int64_t)b * a.out_stride + (int64_t)hq0 * kHeadDim + i] = 0.0f;
-    if (threadIdx.x == 0 && a.dev_err)
-      atomicOr(a.dev_err, GKV_DEVERR_LENGTH);
+  int t0, n;
+  if (!exact_row(a, b, hq0, t0, n))
+    return;
+  if (n <= a.one_tile_n) { // (the host bound may be far above a row's own context)
+    exact_one_tile<false>(a, lds, s_sum, b, g, hq0, t0, n);
     return;
   }
   // a window layer's cache is a ring of window slots (n <= ring: position j of
@@ -209,7 +332,7 @@ __global__ __launch_bounds__(64 * kExactMaxWaves) void attention_exact_kernel(Ex
   // Items of one 64-position tile and up to 8 heads, fewer heads where there
   // would be fewer items than waves (a window, a short context).
   const int tiles = (n + kExactTile - 1) / kExactTile;
-  int hg = 8;
+  int hg = kLite ? 4 : 8;
   while (hg > 1 && tiles * ((hc + hg - 1) / hg) < n_waves)
     hg >>= 1;
   const int n_hg = (hc + hg - 1) / hg;
@@ -218,14 +341,14 @@ __global__ __launch_bounds__(64 * kExactMaxWaves) void attention_exact_kernel(Ex
     const int j = tile * kExactTile + lane;
     const float *kr = kbase + (int64_t)slot_of(min(j, n - 1)) * kv_dim;
     const int nh = min(hg, hc - h);
-    if (nh > 4)
-      exact_scores<8>(kr, qs, h, hc, j, n, att, a.att_row);
+    if (!kLite && nh > 4)
+      exact_scores<8, false>(kr, qs, h, hc, j, n, att, a.att_row);
     else if (nh > 2)
-      exact_scores<4>(kr, qs, h, hc, j, n, att, a.att_row);
+      exact_scores<4, false>(kr, qs, h, hc, j, n, att, a.att_row);
     else if (nh == 2)
-      exact_scores<2>(kr, qs, h, hc, j, n, att, a.att_row);
+      exact_scores<2, !kLite>(kr, qs, h, hc, j, n, att, a.att_row);
     else
-      exact_scores<1>(kr, qs, h, hc, j, n, att, a.att_row);
+      exact_scores<1, !kLite>(kr, qs, h, hc, j, n, att, a.att_row);
   }
   __syncthreads();
 
@@ -326,113 +449,22 @@ __global__ __launch_bounds__(64 * kExactMaxWaves) void attention_exact_kernel(Ex
           acc = __fmaf_rn(x[i], v[(r + e + i) * kHeadDim], acc);
       }
     }
+    if (r + 8 <= m_t) {
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const f32x4 x = *(const f32x4 *)&w[c * R + r + e];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          acc = __fmaf_rn(x[i], v[(r + e + i) * kHeadDim], acc);
+      }
+      r += 8;
+    }
     for (; r < m_t; r++)
       acc = __fmaf_rn(w[c * R + r], v[r * kHeadDim], acc);
   }
   wait_vmcnt<0>(); // no load may still write into LDS when the workgroup ends
   if (wave < hc)
     a.out[(int64_t)b * a.out_stride + (int64_t)(hq0 + wave) * kHeadDim + lane] = acc;
-}
-
-// Short contexts (the rule is at kExactShort): one wave per head, K and V through one
-// LDS tile of 64 positions (65-float rows so that lane t reading row t meets no
-// bank conflict).
-__global__ __launch_bounds__(1024) void attention_exact_short_kernel(ExactAttnArgs a) {
-  extern __shared__ float lds[];
-  __shared__ double s_sum[16];
-  const int b = blockIdx.x;
-  const int g = blockIdx.y / a.n_chunks;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int h = g * a.G + (blockIdx.y % a.n_chunks) * a.hc + wave;
-  const int kv_dim = a.n_kv_heads * kHeadDim;
-  float *kt = lds;                                      // [64][65]
-  float *qs = kt + kExactTile * kExactRow;              // [hc][64]
-  float *att = qs + a.hc * kHeadDim + wave * (a.n_cap + 1); // this head's scores
-
-  const int p = a.positions ? a.positions[b] : a.pos;
-  const int t0 = a.window > 0 ? max(0, p - a.window + 1) : 0;
-  const int n = p - t0 + 1;
-  // a position the cache cannot hold (full layer: p >= slots) or beyond the
-  // host bound: output zeros and the length flag (uniform per workgroup)
-  if (p < 0 || n > a.n_cap || (a.window == 0 && p >= a.slots)) {
-    a.out[(int64_t)b * a.out_stride + (int64_t)h * kHeadDim + lane] = 0.0f;
-    if (threadIdx.x == 0 && a.dev_err)
-      atomicOr(a.dev_err, GKV_DEVERR_LENGTH);
-    return;
-  }
-  const int ring = a.window; // a window layer's cache is a ring of window slots
-  const float *kbase = a.kc + (int64_t)b * a.slots * kv_dim + (int64_t)g * kHeadDim;
-  const float *vbase = a.vc + (int64_t)b * a.slots * kv_dim + (int64_t)g * kHeadDim;
-  qs[wave * kHeadDim + lane] = a.q[(int64_t)b * a.q_stride + (int64_t)h * kHeadDim + lane];
-
-  // scores: (float)((sum_i (double)(q_i * k_i)) / 8), products rounded to fp32
-  const double scale = (double)__fsqrt_rn((float)kHeadDim);
-  for (int tile = 0; tile < n; tile += kExactTile) {
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < kExactTile * kHeadDim; idx += blockDim.x) {
-      const int r = idx >> 6, c = idx & 63, j = tile + r;
-      if (j < n) {
-        const int t = t0 + j;
-        const int slot = ring > 0 ? t % ring : t;
-        kt[r * kExactRow + c] = kbase[(int64_t)slot * kv_dim + c];
-      }
-    }
-    __syncthreads();
-    const int j = tile + lane;
-    if (j < n) {
-      double s = 0.0;
-      for (int i = 0; i < kHeadDim; i++)
-        s = __dadd_rn(s, (double)__fmul_rn(qs[wave * kHeadDim + i], kt[lane * kExactRow + i]));
-      att[j] = (float)__ddiv_rn(s, scale);
-    }
-  }
-  if (lane == 0)
-    att[n] = a.sinks[h];
-  __syncthreads();
-
-  // softmax over att[0..n] (run.cpp:335-353): the max (exact in any order),
-  // expf((float)((double)x - max)), the fp64 sum in index order, the quotients
-  float m = -INFINITY;
-  for (int j = lane; j <= n; j += 64)
-    m = fmaxf(m, att[j]);
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1)
-    m = fmaxf(m, __shfl_xor(m, off));
-  const double md = (double)m;
-  for (int j = lane; j <= n; j += 64)
-    att[j] = expf_cpu_exact((float)__dsub_rn((double)att[j], md));
-  __syncthreads();
-  if (lane == 0) {
-    double s = 0.0;
-    for (int j = 0; j <= n; j++)
-      s = __dadd_rn(s, (double)att[j]);
-    s_sum[wave] = s;
-  }
-  __syncthreads();
-  const double sum = s_sum[wave];
-  for (int j = lane; j <= n; j += 64)
-    att[j] = (float)__ddiv_rn((double)att[j], sum);
-  __syncthreads();
-
-  // out[d] = fma(w_t, v_t[d], out[d]) over t in order; the V rows go through
-  // the K tile's LDS, 64 positions at a time, read once for the hc heads
-  float acc = 0.0f;
-  for (int tile = 0; tile < n; tile += kExactTile) {
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < kExactTile * kHeadDim; idx += blockDim.x) {
-      const int r = idx >> 6, c = idx & 63, j = tile + r;
-      if (j < n) {
-        const int t = t0 + j;
-        const int slot = ring > 0 ? t % ring : t;
-        kt[r * kExactRow + c] = vbase[(int64_t)slot * kv_dim + c];
-      }
-    }
-    __syncthreads();
-    const int m_t = min(kExactTile, n - tile);
-    for (int r = 0; r < m_t; r++)
-      acc = __fmaf_rn(att[tile + r], kt[r * kExactRow + lane], acc);
-  }
-  a.out[(int64_t)b * a.out_stride + (int64_t)h * kHeadDim + lane] = acc;
 }
 
 // run.cpp's apply_rotary_emb on heads 0..n_heads-1 of each row, in place.
@@ -588,33 +620,43 @@ extern "C" int gkv_attention_exact(void *stream, int32_t B, int32_t n_q_heads,
   void (*fn)(ExactAttnArgs);
   const int64_t wgs = (int64_t)B * n_kv_heads * a.n_chunks;
   int short_cap = kExactShort;
-  if (wgs > kExactMany && hc >= 3)
-    short_cap = wgs <= kExactVeryMany ? kExactShortMany : kExactShortVeryMany;
-  else if (wgs > kExactTwo && wgs <= kExactMany && hc >= 5)
-    short_cap = hc > kExactMaxWaves / 2 && hc < kExactMaxWaves ? kExactShortTwoOdd : kExactShortTwo;
+  if (wgs > kExactTwo && wgs <= kExactMany && hc >= 5)
+    short_cap = kExactShortTwo;
+  else if (wgs > kExactMany && wgs <= kExactFour && hc >= 5 && hc <= 8)
+    short_cap = kExactShortFour;
   if (n_cap <= short_cap) {
     lds = kFixed - 256 + (size_t)hc * (kHeadDim + n_cap + 1) * sizeof(float);
     threads = 64 * hc;
     fn = attention_exact_short_kernel;
   } else {
     a.att_row = (n_cap + 1 + 3) / 4 * 4;
-    // waves: a whole number per head, at most one per head and 64-position tile
     const int tiles = (n_cap + kExactTile - 1) / kExactTile;
-    a.parts = std::max(1, std::min(kExactMaxWaves / hc, tiles));
-    // The V ring: 4 stages of 64 rows where the LDS has room
-    // and the loading waves need at most 16 loads each, else of 16 rows, which
-    // kFixed always holds (then in the place of the sums' fp64 values).
     const size_t rows_bytes = (size_t)hc * (kHeadDim + a.att_row) * sizeof(float);
     const size_t dbl_bytes = (size_t)hc * 128 * sizeof(double);
     auto ring_bytes = [](int rows) { return (size_t)4 * rows * kHeadDim * sizeof(float); };
+    // The V ring's smallest form (16 rows a stage, in the place of the sums' fp64
+    // values) is what kFixed always holds.
+    const size_t least = rows_bytes + std::max(ring_bytes(16), dbl_bytes);
+    const bool lite = wgs > kExactTwo && 2 * (least + 256) <= lim;
+    // waves: a whole number per head, at most one per head and 64-position tile
+    const int most = lite && wgs > kExactFour && hc <= kExactMaxWaves / 2 ? kExactMaxWaves / 2
+                                                                          : kExactMaxWaves;
+    a.parts = std::max(1, std::min(most / hc, tiles));
     const int waves = hc * a.parts, n_load = waves > hc ? waves - hc : waves;
-    const size_t room = lim - 256 - rows_bytes; // (256: the static arrays)
-    a.v_rows = n_load >= 4 && ring_bytes(64) + dbl_bytes <= room ? 64 : 16;
+    // The ring's stages: as many rows (at most 16 loads a loading wave) as leave room
+    // for the workgroups a CU is to hold (256: the static arrays)
+    const size_t hold = !lite ? 1 : most == kExactMaxWaves ? 2 : std::min<size_t>(4, lim / (least + 256));
+    const size_t room = lim / hold - 256 - rows_bytes;
+    a.v_rows = 64;
+    while (a.v_rows > 16 && (a.v_rows > 16 * n_load || std::max(ring_bytes(a.v_rows), dbl_bytes) > room))
+      a.v_rows -= 8;
     a.v_early = ring_bytes(a.v_rows) + dbl_bytes <= room;
     lds = rows_bytes + (a.v_early ? ring_bytes(a.v_rows) + dbl_bytes
                                   : std::max(ring_bytes(a.v_rows), dbl_bytes));
+    const int one_tile_floats = (int)(lds / sizeof(float)) - kExactTile * kExactRow - hc * kHeadDim;
+    a.one_tile_n = std::min(kExactShort, one_tile_floats / hc - 1);
     threads = 64 * waves;
-    fn = attention_exact_kernel;
+    fn = lite ? attention_exact_kernel<true> : attention_exact_kernel<false>;
   }
   if (lds > 64 * 1024 &&
       hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize,

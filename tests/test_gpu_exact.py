@@ -120,16 +120,23 @@ def _attention_case(seed, B, Hq, Hkv, lens_lo, lens_hi, window=0, slots=None):
     ("tiles", 3, 3, 1, 255, 257, 0),             # 64-position tiles full, one short, one over
     ("group16_wide", 2, 16, 1, 2100, 2300, 0),   # 16 heads at once, 16-row V stages
     ("lds_full", 1, 8, 1, 4400, 4400, 0),        # the V ring in the sums' place
-    ("many", 65, 64, 8, 1, 512, 0),              # just over 512 workgroups: the one-tile form
-    ("many_long", 65, 24, 8, 500, 513, 0),       # ... up to 512 positions, 3 heads a group
-    ("very_many", 257, 32, 8, 1, 640, 0),        # over 2048 workgroups: up to 640 positions
-    ("very_many_long", 257, 24, 8, 1, 641, 0),   # one more: the long form
-    ("many_two_heads", 65, 16, 8, 1, 300, 0),    # two heads a group: the long form
-    ("second_round", 33, 64, 8, 1, 256, 0),      # just over 256 workgroups: one-tile up to 256
-    ("second_round_long", 33, 40, 8, 1, 257, 0),  # one position more, 5 heads: the long form
-    ("second_round_few", 33, 32, 8, 200, 256, 0),  # 4 heads a group: the long form
-    ("second_round_odd", 257, 10, 1, 1, 320, 0),   # 10 heads, no idle waves: one-tile up to 320
-    ("second_round_odd_long", 257, 9, 1, 300, 321, 0),
+    ("ring40", 1, 8, 1, 3600, 3600, 0),          # 40-row V stages
+    ("two_short", 33, 64, 8, 1, 256, 0),         # just over 256 workgroups: one-tile up to 256
+    ("two_per_cu", 33, 64, 8, 1, 257, 0),        # ... then 64 registers
+    ("two_per_cu_5", 33, 40, 8, 1, 257, 0),      # 5 heads, 15 waves
+    ("two_per_cu_4", 33, 32, 8, 200, 256, 0),    # 4 heads, 16 waves
+    ("two_per_cu_10", 257, 10, 1, 1, 320, 0),    # 10 heads, a wave each, no other to load
+    ("two_per_cu_9", 257, 9, 1, 300, 321, 0),
+    ("two_per_cu_ring", 33, 64, 8, 1, 900, 320),  # 320-slot rings, some rows short of 192
+    ("two_per_cu_24", 33, 64, 8, 100, 1500, 0),  # 24-row V stages
+    ("many_short", 65, 64, 8, 1, 300, 0),        # 513 .. 1024 workgroups: one-tile up to 300
+    ("many_short_edge", 65, 64, 8, 200, 301, 0),
+    ("many", 65, 64, 8, 1, 512, 0),
+    ("many_long", 65, 24, 8, 500, 513, 0),       # 3 heads a group
+    ("very_many", 257, 32, 8, 1, 640, 0),        # over 1024 workgroups: 8 waves each
+    ("very_many_long", 257, 24, 8, 1, 641, 0),   # 3 heads, 6 waves
+    ("very_many_12", 257, 48, 4, 1, 300, 0),     # 12 heads, 12 waves
+    ("many_two_heads", 65, 16, 8, 1, 300, 0),    # two heads a group
 ])
 def test_attention_exact_bit_exact(gkv, cuda, name, B, Hq, Hkv, lo, hi, window):
     import torch
@@ -146,6 +153,51 @@ def test_attention_exact_bit_exact(gkv, cuda, name, B, Hq, Hkv, lo, hi, window):
     torch.cuda.synchronize()
     assert int(err.item()) == 0
     assert_bits_equal(out.cpu().numpy().reshape(B, Hq, D), want, name)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,bound,window", [
+    (5, 16, 2, 1000, 0), (40, 64, 8, 700, 0), (40, 64, 8, 1600, 0), (300, 8, 1, 4000, 0),
+    (130, 32, 8, 900, 0), (300, 16, 4, 2500, 0), (70, 64, 8, 5000, 304)])
+def test_attention_exact_bound_far_above_the_contexts(gkv, cuda, B, Hq, Hkv, bound, window):
+    """Rows of 1 .. 300 positions (both sides of the one-tile form's 192) under a host
+    bound that picks the long forms."""
+    import torch
+    pos, q, kc, vc, sinks, slots = _attention_case(bound + B, B, Hq, Hkv, 1, 300, window)
+    pos[:2] = 191, 192
+    kc, vc = np.nan_to_num(kc, nan=0.25), np.nan_to_num(vc, nan=-0.25)
+    want = O.decode_attention(q, kc, vc, pos, sinks, window=window, ring=window)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    out = torch.full((B, Hq * D), float("nan"), device=cuda)
+    err = torch.zeros(1, dtype=torch.int32, device=cuda)
+    print(f"attention_exact B={B} Hq={Hq} Hkv={Hkv} bound={bound} window={window}", flush=True)
+    gkv.attention_exact(d(q.reshape(B, Hq * D)), Hq, Hkv, d(kc.reshape(B, slots, Hkv * D)),
+                        d(vc.reshape(B, slots, Hkv * D)), d(sinks), out, positions=d(pos),
+                        max_pos=bound, window=window, dev_err=err)
+    torch.cuda.synchronize()
+    assert int(err.item()) == 0
+    assert_bits_equal(out.cpu().numpy().reshape(B, Hq, D), want, f"bound {bound}")
+
+
+@pytest.mark.parametrize("n", [100, 300])
+def test_attention_exact_at_any_float(gkv, cuda, n):
+    """Queries, caches and outputs one float off a 16-byte boundary, in both forms."""
+    import torch
+    B, Hq, Hkv = 3, 16, 2
+    pos, q, kc, vc, sinks, slots = _attention_case(n, B, Hq, Hkv, 1, n)
+    want = O.decode_attention(q, kc, vc, pos, sinks)
+
+    def off_by_one(a, *shape):
+        buf = torch.full((a.size + 1,), float("nan"), device=cuda)
+        buf[1:] = torch.from_numpy(np.ascontiguousarray(a)).reshape(-1).to(cuda)
+        return buf[1:].view(*shape)
+
+    out = off_by_one(np.zeros(B * Hq * D, np.float32), B, Hq * D)
+    print(f"attention_exact off by one float, {n} positions", flush=True)
+    gkv.attention_exact(off_by_one(q, B, Hq * D), Hq, Hkv, off_by_one(kc, B, slots, Hkv * D),
+                        off_by_one(vc, B, slots, Hkv * D), off_by_one(sinks, Hq), out,
+                        positions=torch.from_numpy(pos).to(cuda), max_pos=n - 1)
+    torch.cuda.synchronize()
+    assert_bits_equal(out.cpu().numpy().reshape(B, Hq, D), want, f"{n} positions")
 
 
 def test_attention_exact_one_position_and_flags(gkv, cuda):
