@@ -393,3 +393,38 @@ def test_rows_four_gigabytes_apart(gkv, cuda):
     scale = (x.double().abs() @ w.double().abs().t()).cpu().numpy()
     for o in out:
         assert (np.abs(o.cpu().numpy() - ref) <= 2e-5 * scale + 1e-6).all()
+
+
+@pytest.mark.parametrize("rows", [5, 40, 150, 500, 700, 1000, 1700])
+def test_rows_bias_and_tables_at_any_float(gkv, cuda, rows):
+    """The fp32 rows, the bias and the angle tables one float off a 16-byte boundary
+    and with an odd row stride, in every launch shape of 5120 columns: the same
+    rows and cache bytes as aligned ones, and nothing written beside them."""
+    import torch
+    rng = np.random.default_rng(rows)
+    case = QkvCase(rows, 64, 8, 64, lens=rng.integers(1, 40, rows))
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)  # noqa: E731
+    cos, sin = gkv.rope_table(int(case.lens.max()) + 1)
+    x, w = t(case.x).to(torch.bfloat16), t(case.w).to(torch.bfloat16)
+    lens, table = t(case.lens), t(case.table)
+
+    def off_by_one(a):
+        buf = torch.zeros(a.size + 1, device=cuda)
+        buf[1:] = t(a.reshape(-1))
+        return buf[1:]
+
+    got = []
+    for shifted in (False, True):
+        put = off_by_one if shifted else t
+        buf = torch.full((rows * (case.N + 3) + 1,), float("nan"), device=cuda)
+        out = buf[int(shifted):].as_strided((rows, case.N), (case.N + 3 * shifted, 1))
+        k = torch.zeros(case.NB, case.Hkv, 16 * D, dtype=torch.int16, device=cuda)
+        v = torch.zeros_like(k)
+        gkv.qkv_append(x, w, put(case.bias), case.Hq, put(cos), put(sin),
+                       gkv.cache_view(k, v, table, case.Hkv), seq_lens=lens, qkv_out=out)
+        torch.cuda.synchronize()
+        assert int(torch.isnan(buf).sum()) == buf.numel() - rows * case.N
+        got.append([z.cpu().numpy() for z in (out.contiguous(), k, v)])
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.int32 if a.dtype == np.float32 else a.dtype),
+                              b.view(np.int32 if b.dtype == np.float32 else b.dtype))
