@@ -55,9 +55,10 @@
 // lane and 32-key step, about 70 other) beside 24 matrix ops. So the scale
 // stands in the exponent's FMA, the rescale test is one compare of the row sum,
 // the query is split into its pieces two values at a time, and a quantized V's
-// mask and power of two go into its scales: 8 chunks of 100 .. 700 tokens after
-// 1536 cached ones, int8 V, 251 -> 237 us; 64 prompts of 64 .. 512 tokens 228
-// -> 222 us (full layer), 189 -> 185 us (window).
+// power of two goes into its scales. The attention alone, both forms timed in turn
+// (events, medians of 9): 8 chunks of 100 .. 700 tokens after 1536 cached ones 231 -> 216
+// us with int8 V, 254 -> 249 with the e4m3 cache, 216 -> 215 with bf16; 64 prompts of
+// 64 .. 512 tokens 194 -> 190 us (full layer), 162 -> 158 us (window).
 #include "gkv_device.hpp"
 #include "lds_dma.hpp"
 

@@ -21,12 +21,13 @@
 // alike -- both halves of a RoPE pair. The operands of a slice are read from
 // LDS into registers among the matrix ops of the slice before, and one
 // barrier per stage both publishes the next stage and frees this one.
-// What bounds it: with many rows the matrix cores (9507 rows: 243 us = 1154
+// What bounds it: with many rows the matrix cores (9507 rows: 249 us = 1126
 // TFLOP/s, of which 200 in the K loop, the fp32 rows' 195 MB most of the rest;
 // 128 x 128 tiles without the operand buffering, the workgroups of an XCD
-// spread over all row blocks: 402), at 512 rows the latency of the operand
-// stream (1.2 us from a load's issue to its data, whatever the tile), with few
-// rows the chain of K steps.
+// spread over all row blocks: 372 in turn with it), at 512 rows the operands' way
+// into LDS (640 tiles bring 471 MB; under that load an operand takes 1.2 us from
+// its load's issue) and the third tile on half the CUs, with few rows the chain of
+// K steps.
 //
 // Placement of each row (its sequence, position, slot and block) is loaded by
 // the first waves in three dependent hops of direct-to-LDS loads spread over the
