@@ -1871,11 +1871,12 @@ template <int R>
 static void launch_fused_ring(const DecodeArgs &a, const AppendArgs &ap, int mode, dim3 grid,
                               dim3 block, hipStream_t s) {
   if (a.kv_fp8) {
-    // The e4m3 stream is bound by its waves' instructions (half the bytes per
-    // step, the same math plus the code conversions): two waves per SIMD, one
-    // kv head each, cover each other's dependency chains; at 256 registers
-    // the ring is 2 steps deep (3 would spill). Measured 125.1 against
-    // 130.9 us at config 2; the bf16 and int8-V streams, bound by their
+    // One wave per SIMD runs the e4m3 stream at the pace of its own instructions
+    // (half the bytes per step, the same math plus the code conversions: ready
+    // but not issued 10% of its cycles, bf16's 48%). Two, one kv head each, cover
+    // each other's dependency chains and execute in 70% of the SIMD's cycles;
+    // at 256 registers the ring is 2 steps deep (3 would spill). Measured 125.1
+    // against 130.9 us at config 2; the bf16 and int8-V streams, bound by their
     // loads, measured level or slower this way.
     hipLaunchKernelGGL((decode_fused_kernel<2, 2, false, kMaxSplitWaves>), grid,
                        dim3(64 * std::min(kMaxSplitWaves, a.n_kv_heads)), 0, s, a, ap, mode);

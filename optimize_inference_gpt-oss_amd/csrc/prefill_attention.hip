@@ -56,9 +56,9 @@
 // stands in the exponent's FMA, the rescale test is one compare of the row sum,
 // the query is split into its pieces two values at a time, and a quantized V's
 // power of two goes into its scales. The attention alone, both forms timed in turn
-// (events, medians of 9): 8 chunks of 100 .. 700 tokens after 1536 cached ones 231 -> 216
-// us with int8 V, 254 -> 249 with the e4m3 cache, 216 -> 215 with bf16; 64 prompts of
-// 64 .. 512 tokens 194 -> 190 us (full layer), 162 -> 158 us (window).
+// (events, two runs): 8 chunks of 100 .. 700 tokens after 1536 cached ones 231 -> 216
+// us with int8 V, 254 -> 249 with the e4m3 cache, level (216) with bf16; 64 prompts of
+// 64 .. 512 tokens 192 - 194 -> 187 - 190 us (full layer), 160 - 162 -> 158 - 160 (window).
 #include "gkv_device.hpp"
 #include "lds_dma.hpp"
 

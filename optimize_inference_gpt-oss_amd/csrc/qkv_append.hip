@@ -22,7 +22,7 @@
 // LDS into registers among the matrix ops of the slice before, and one
 // barrier per stage both publishes the next stage and frees this one.
 // What bounds it: with many rows the matrix cores (9507 rows: 249 us = 1126
-// TFLOP/s, of which 200 in the K loop, the fp32 rows' 195 MB most of the rest;
+// TFLOP/s, 243 - 256 by GPU, of which 200 in the K loop, the fp32 rows' 195 MB most of the rest;
 // 128 x 128 tiles without the operand buffering, the workgroups of an XCD
 // spread over all row blocks: 372 in turn with it), at 512 rows the operands' way
 // into LDS (640 tiles bring 471 MB; under that load an operand takes 1.2 us from
