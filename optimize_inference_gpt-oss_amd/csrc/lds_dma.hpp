@@ -76,24 +76,27 @@ __device__ __forceinline__ void dma16_s(const void *base, uint32_t byte_off, voi
 
 // dma16_s in a loop whose LDS and global addresses are kept as numbers: the
 // LDS byte address of the wave's 1 KB (the low half of a generic pointer into
-// LDS is its LDS address) and the base both wave-uniform.
+// LDS is its LDS address) and the base both wave-uniform. M0 is an operand, which
+// the compiler sets, instead of saved and restored around the load. kSalu: the
+// base comes from scalar arithmetic on uniform values, so the one wait state that
+// a load into LDS needs after a write of M0 is enough; else it may come
+// from v_readfirstlane, and the asm brings all five. (9507 projection rows, in turn
+// with loads of two wait states that leave M0 changed: 2% slower with the five and
+// M0 saved in every form, 243.0 / 248.0 us; level so, 252.6 / 252.4 on another GPU.)
 __device__ __forceinline__ uint32_t lds_addr(const void *p) {
   return (uint32_t)(uintptr_t)(lds_ptr)p;
 }
+template <bool kSalu>
 __device__ __forceinline__ void dma16_at(const void *base, uint32_t byte_off, uint32_t lds) {
   const uint64_t b = (uint64_t)(uintptr_t)base;
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
   const uint64_t sb = ((uint64_t)hi << 32) | lo;
   const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane(lds);
-  uint32_t saved;
-  asm volatile("s_mov_b32 %0, m0\n\t"
-               "s_mov_b32 m0, %3\n\t"
-               "s_nop 2\n\t"
-               "global_load_lds_dwordx4 %1, %2\n\t"
-               "s_mov_b32 m0, %0" // (M0 is reserved: no clobber may name it)
-               : "=&s"(saved)
-               : "v"(byte_off), "s"(sb), "s"(m)
+  asm volatile("s_nop %3\n\t"
+               "global_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(byte_off), "s"(sb), "{m0}"(m), "n"(kSalu ? 0 : 4)
                : "memory");
 }
 

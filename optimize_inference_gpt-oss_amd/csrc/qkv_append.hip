@@ -402,10 +402,10 @@ __global__ __launch_bounds__(64 * kWM * (kGN / 64) * kWK) void qkv_append_kernel
     if constexpr (kWide)
       dma16(base + off[i], &stage[st * kStageElems + u * 512]);
     else if (kOneW && !is_x) // 64 columns on, or the last 64
-      dma16_at(base + (int64_t)min(64 * (i - kXC / kNW), (a.N - 64 - n0)) * a.K * 2,
+      dma16_at<kEven>(base + (int64_t)min(64 * (i - kXC / kNW), (a.N - 64 - n0)) * a.K * 2,
                off[kXC / kNW], dst);
     else
-      dma16_at(base, off[i], dst);
+      dma16_at<kEven>(base, off[i], dst); // (kEven: no part of the base is the wave's)
   };
   auto dma_chunk = [&](int kc, int st) {
 #pragma unroll
